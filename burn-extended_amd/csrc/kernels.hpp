@@ -279,6 +279,7 @@ struct DequantArgs {
   uint64_t rows, cols, bpr, gpr;
   int ue8_offset;
   int out_bf16;
+  int vec;  // out 16-byte aligned (set by launch_dequant)
 };
 
 size_t router_lds_bytes(uint32_t tb, uint32_t Dpad);
