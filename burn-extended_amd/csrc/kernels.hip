@@ -575,13 +575,14 @@ __device__ __forceinline__ uint32_t half_wave_incl_scan(uint32_t v) {
 }
 
 // Exclusive prefix sums over the experts e < E (E <= 256) of their entry counts c_e, of
-// [c_e > 0] and of ceil(c_e / kGemmTok), for thread e (threads 0 .. 255 of a workgroup of at least
+// [c_e > 0] and of ceil(c_e / 2^tsh), for thread e (threads 0 .. 255 of a workgroup of at least
 // 256): wave scans, then the totals of the waves below from LDS (tot_l: 12 ints).  Called by
 // every thread of the workgroup (two barriers); threads from 256 on get zeros.
-__device__ void expert_prefix(const int32_t *cnt, uint32_t E, int32_t *tot_l, int32_t &off, int32_t &ra, int32_t &toff) {
+__device__ void expert_prefix(const int32_t *cnt, uint32_t E, uint32_t tsh, int32_t *tot_l, int32_t &off, int32_t &ra,
+                              int32_t &toff) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
   const int32_t c = (tid < E && tid < kMaxExperts) ? cnt[tid] : 0;
-  const uint32_t v0 = (uint32_t)c, v1 = c > 0 ? 1u : 0u, v2 = (uint32_t)((c + (int32_t)kGemmTok - 1) / (int32_t)kGemmTok);
+  const uint32_t v0 = (uint32_t)c, v1 = c > 0 ? 1u : 0u, v2 = ((uint32_t)c + (1u << tsh) - 1u) >> tsh;
   const uint32_t i0 = wave_incl_scan(v0), i1 = wave_incl_scan(v1), i2 = wave_incl_scan(v2);
   if (w < 4u && lane == 63u) {
     tot_l[3u * w] = (int32_t)i0;
@@ -701,7 +702,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_kernel(TopkArgs a) {
 // ---------------------------------------------------------------------------------------------
 __device__ void block_dispatch(const int32_t *idx, uint32_t n, uint32_t K, uint32_t E, int32_t *seg_off,
                                int32_t *perm, int32_t *pos_of, int32_t *active, int32_t *num_active,
-                               int32_t *exrec, int32_t *tile_off, int32_t *lds) {
+                               int32_t *exrec, int32_t *tile_off, uint32_t tsh, int32_t *lds) {
   const uint32_t tid = threadIdx.x, nth = blockDim.x, words = nth >> 5;  // 32 words: nth = 1024
   int32_t *cnt = lds, *base = lds + E;
   uint32_t *bm = (uint32_t *)(lds + 2 * E);
@@ -718,7 +719,7 @@ __device__ void block_dispatch(const int32_t *idx, uint32_t n, uint32_t K, uint3
   __syncthreads();
   // exclusive scans and active list (expert e by thread e)
   int32_t off, ra, toff;
-  expert_prefix(cnt, E, tot_l, off, ra, toff);
+  expert_prefix(cnt, E, tsh, tot_l, off, ra, toff);
   if (tid < E) {
     const uint32_t e = tid;
     if (tile_off) tile_off[e] = toff;
@@ -734,7 +735,7 @@ __device__ void block_dispatch(const int32_t *idx, uint32_t n, uint32_t K, uint3
     }
     if (e + 1 == E) {
       seg_off[E] = off + cnt[e];
-      if (tile_off) tile_off[E] = toff + (cnt[e] + (int32_t)kGemmTok - 1) / (int32_t)kGemmTok;
+      if (tile_off) tile_off[E] = toff + (int32_t)(((uint32_t)cnt[e] + (1u << tsh) - 1u) >> tsh);
       const int32_t na = ra + (cnt[e] > 0);
       *num_active = na;
       lds[4 * E + 2 * E * words] = na;
@@ -869,7 +870,7 @@ __global__ __launch_bounds__(kDispatchChunk) void dispatch_wide_kernel(DispatchA
   __syncthreads();
   // exclusive scans over experts (expert e by thread e)
   int32_t off, ra, toff;
-  expert_prefix(call, E, tot_l, off, ra, toff);
+  expert_prefix(call, E, a.tile_shift, tot_l, off, ra, toff);
   if (tid < E) {
     const uint32_t e = tid;
     segs[e] = off;
@@ -886,7 +887,7 @@ __global__ __launch_bounds__(kDispatchChunk) void dispatch_wide_kernel(DispatchA
       }
       if (e + 1 == E) {
         a.seg_off[E] = off + call[e];
-        if (a.tile_off) a.tile_off[E] = toff + (call[e] + (int32_t)kGemmTok - 1) / (int32_t)kGemmTok;
+        if (a.tile_off) a.tile_off[E] = toff + (int32_t)(((uint32_t)call[e] + (1u << a.tile_shift) - 1u) >> a.tile_shift);
         const int32_t na = ra + (call[e] > 0);
         *a.num_active = na;
         for (uint32_t e3 = (uint32_t)na; e3 < E; ++e3) a.active[e3] = -1;
@@ -916,7 +917,7 @@ __global__ __launch_bounds__(kDispatchChunk) void dispatch_wide_kernel(DispatchA
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_kernel(DispatchArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   block_dispatch(a.topk_idx, a.n, a.K, a.E, a.seg_off, a.perm, a.pos_of, a.active, a.num_active, a.exrec,
-                 a.tile_off, (int32_t *)smem);
+                 a.tile_off, a.tile_shift, (int32_t *)smem);
 }
 
 // ---------------------------------------------------------------------------------------------

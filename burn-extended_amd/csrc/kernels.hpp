@@ -83,9 +83,10 @@ struct DispatchArgs {
   const int32_t *topk_idx;
   int32_t *seg_off, *perm, *pos_of, *active, *num_active;
   int32_t *exrec;     // [E, kRecWords]
-  int32_t *tile_off;  // [E + 1] prefix of ceil(M_e / kGemmTok), or null
+  int32_t *tile_off;  // [E + 1] prefix of ceil(M_e / 2^tile_shift), or null
   int32_t *chunk_cnt; // [ceil(n / kDispatchChunk), E] scratch of the multi-workgroup dispatch
   uint32_t n, K, E;
+  uint32_t tile_shift;  // log2 of the tokens per tile of tile_off
 };
 
 // One expert projection over the tiled MXFP4 layout (see the expert_gemv comment in kernels.hip).
@@ -214,6 +215,28 @@ struct GemmArgs {
   QRows act;               // gate_up output: SwiGLU rows in segment order, quantised
   uint32_t act_feats;      // gate_up: F (features written; [F, act.kq) zero-filled)
   uint16_t *out;           // down: token-major slot rows [n*k, out_stride] bf16
+  uint32_t out_stride;
+  float alpha, limit;
+};
+
+// Grouped expert GEMM on bf16 MFMA (expert_tile_kernel): operands and roundings of the expert GEMV,
+// work items of t.tok routed tokens of one expert x 64 t.row_tiles weight rows.
+struct TileShape {
+  uint32_t row_tiles, tok;  // 16-row tiles per wave, tokens
+};
+constexpr TileShape kTileLarge = {4, 64}, kTileSmall = {2, 32};
+struct TileArgs {
+  const uint8_t *wb, *ws;  // tiled MXFP4 codes; scales in the GEMM's copy (as GemmArgs)
+  uint64_t wb_estride, ws_estride;
+  const float *bias;       // [E, rows_p]
+  uint32_t bias_estride;
+  uint32_t nrt, nb, kt, out_rows;  // out_rows: gate_up F features, down D rows
+  uint32_t nrb;            // 64 row_tiles-row blocks per expert
+  const int32_t *seg_off, *tile_off, *perm;
+  uint32_t E, topk;
+  const void *brows;       // gate_up xn [n, bstride] (x dtype), down act [n*k, bstride] f32 (segment order)
+  uint32_t bstride;
+  float *out;              // gate_up: act [n*k, out_stride] (segment order); down: token-major slot rows
   uint32_t out_stride;
   float alpha, limit;
 };
@@ -360,6 +383,8 @@ hipError_t configure_fused_kernels();
 hipError_t launch_gemm(const GemmArgs &a, bool gate_up, uint32_t grid, hipStream_t s);
 hipError_t configure_gemm_kernels();
 size_t gemm_lds_bytes();
+hipError_t launch_tile(const TileArgs &a, const TileShape &t, int nt, bool gate_up, bool x_bf16, uint32_t grid, hipStream_t s);
+hipError_t configure_tile_kernels();
 hipError_t launch_dequant(const DequantArgs &a, hipStream_t s);
 hipError_t configure_kernels();
 

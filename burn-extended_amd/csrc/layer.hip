@@ -339,17 +339,36 @@ struct WsLayout {
   bool gemm;                        // the grouped-GEMM regions are present
 };
 
-// bf16 batches of at least kGemmMinTokens tokens with at least kGemmMinPerExpert routed tokens per
-// expert on average run the grouped GEMM; the others, and every f32 batch (the GEMM's two activation
-// terms carry about 2^-6 relative precision), run the expert GEMVs.  Measured per step (us, GEMV
-// against GEMM, D = F = 2880, k = 4): E = 32: 145 / 147 at 32 tokens, 175 / 144 at 64, 239 / 155 at
-// 128, 367 / 163 at 256; E = 128: 366 / 390 at 64, 469 / 439 at 128, 438 / 448 at 200, 455 / 461 at
-// 256, 796 / 494 at 512.
+// Batches whose workspace holds the grouped GEMM's regions: from 64 tokens and 4 routed tokens per
+// expert on.
 constexpr uint64_t kGemmMinTokens = 64;
 constexpr uint64_t kGemmMinPerExpert = 4;
-inline bool use_gemm_path(const burnext_moe_layer &L, uint64_t n) {
+inline bool gemm_regions(const burnext_moe_layer &L, uint64_t n) {
   return n >= kGemmMinTokens && n * L.K >= kGemmMinPerExpert * L.E;
 }
+
+// The expert projections by batch size: up to kSmallRouteMaxTokens tokens the expert GEMVs; beyond, as
+// tiles on bf16 MFMA (tile_gemm.hip: the GEMV's operands and precision), except bf16 batches of
+// kMxMinTokens tokens and kMxMinPerExpert routed tokens per expert, which run the grouped GEMM on the
+// block-scaled MFMA (its two activation terms carry about 2^-6 relative precision: bf16 rows only).
+// Tiles against the grouped GEMM per step, D = F = 2880, k = 4, bf16: E = 32 109 / 134 us at 64 tokens,
+// 125 / 135 at 128, 129 / 136 at 160, 141 / 139 at 200, 162 / 141 at 256; E = 128 322 / 384 at 128, 358 / 398
+// at 200, 400 / 415 at 300, 428 / 428 at 400, 448 / 439 at 512.  Against GEMV passes of 8 .. 14 token rows:
+// E = 32 bf16 98 / 107 us at 17 tokens, 101 / 113 at 45, 108 / 130 at 63, f32 115 / 133 at 17 and 340 / 1085 at
+// 523; E = 128 bf16 278 / 308 at 64, 310 / 376 at 100.
+constexpr uint64_t kMxMinTokens = 192;
+constexpr uint64_t kMxMinPerExpert = 12;
+inline bool use_mx_gemm(const burnext_moe_layer &L, uint64_t n, bool xb) {
+  return xb && n >= kMxMinTokens && n * L.K >= kMxMinPerExpert * L.E;
+}
+static_assert(kMxMinTokens >= kGemmMinTokens && kMxMinPerExpert >= kGemmMinPerExpert, "the GEMM path has its regions");
+
+// Tiles of 32 tokens x 128 rows up to 224 tokens (four workgroups a CU, weights streamed past the
+// caches), of 64 x 256 beyond (half the operand reads and weight conversions per product).  32 x 128
+// against 64 x 256 per step: E = 32 bf16 125 / 133 us at 128 tokens, 141 / 151 at 200, 181 / 162 at 256, f32
+// 170 / 187 at 200, 215 / 204 at 256; E = 128 bf16 278 / 302 at 64, 358 / 363 at 200, 406 / 400 at 300.
+constexpr uint64_t kTileSmallMaxTokens = 224;
+inline TileShape tile_shape(uint64_t n) { return n <= kTileSmallMaxTokens ? kTileSmall : kTileLarge; }
 
 // Codes per row of the GEMM's activation rows over K = cols of a tiled projection (whole 128-wide
 // K-groups): the hi term's bytes; the lo term takes half as many.
@@ -408,7 +427,7 @@ WsLayout ws_layout(const burnext_moe_layer &L, uint64_t n) {
   w.exrec = take((uint64_t)L.E * kRecWords * 4);
   w.perm = take(nk * 4);
   w.pos_of = take(nk * 4);
-  w.gemm = use_gemm_path(L, n);
+  w.gemm = gemm_regions(L, n);
   w.xn = take(n * L.Dp * 4);  // normalised rows, x dtype (f32 size covers both)
   w.act = take(nk * L.Fp * 4);
   if (w.gemm) {
@@ -466,6 +485,9 @@ WsPtrs ws_ptrs(const burnext_moe_layer &L, const WsLayout &w, void *base) {
     p.xq = QRows{b + w.xq[0], b + w.xq[1], b + w.xq[2], b + w.xq[3], qrow_bytes(L.w1), qscale_bytes(L.w1)};
     p.aq = QRows{b + w.aq[0], b + w.aq[1], b + w.aq[2], b + w.aq[3], qrow_bytes(L.w2), qscale_bytes(L.w2)};
   }
+  // (without the grouped GEMM's regions: over the logits, which nothing reads once the top-k is
+  // taken; the dispatch that writes it comes after, and n * E >= E + 1 there)
+  if (!w.gemm) p.tile_off = (int32_t *)p.logits;
   p.perm = (int32_t *)(b + w.perm);
   p.pos_of = (int32_t *)(b + w.pos_of);
   p.act = (float *)(b + w.act);
@@ -612,10 +634,14 @@ burnext_status run_topk(burnext_moe_layer *L, uint64_t n, const float *logits, i
 
 burnext_status run_dispatch(burnext_moe_layer *L, uint64_t n, const int32_t *idx, int32_t *seg_off, int32_t *perm,
                             int32_t *pos_of, int32_t *active, int32_t *num_active, int32_t *exrec,
-                            int32_t *chunk_cnt, hipStream_t s, int32_t *tile_off = nullptr) {
+                            int32_t *chunk_cnt, hipStream_t s, int32_t *tile_off = nullptr,
+                            uint32_t tile_tok = kGemmTok) {
+  static_assert((kGemmTok & (kGemmTok - 1u)) == 0 && (kTileSmall.tok & (kTileSmall.tok - 1u)) == 0 &&
+                    (kTileLarge.tok & (kTileLarge.tok - 1u)) == 0, "tiles of a power of two tokens");
   DispatchArgs da{};
   da.chunk_cnt = chunk_cnt;
   da.tile_off = tile_off;
+  da.tile_shift = (uint32_t)__builtin_ctz(tile_tok);
   da.exrec = exrec;
   da.topk_idx = idx;
   da.seg_off = seg_off;
@@ -787,7 +813,7 @@ burnext_status run_fused(burnext_moe_layer *L, uint64_t n, int nt, bool xb, cons
   return check_launch(launch_fused(a, fg, nt, xb, s), "fused experts launch");
 }
 
-// Grouped-GEMM path (use_gemm_path): router (+ the two-term rows of xn), top-k,
+// Grouped-GEMM path (use_mx_gemm): router (+ the two-term rows of xn), top-k,
 // dispatch (+ token-tile prefix), gate_up GEMM (SwiGLU, quantised act rows), down GEMM (slot rows).
 burnext_status forward_gemm(burnext_moe_layer *L, const void *x, bool xb, uint64_t n, bool norm, const WsPtrs &p,
                             hipStream_t s) {
@@ -829,6 +855,50 @@ burnext_status forward_gemm(burnext_moe_layer *L, const void *x, bool xb, uint64
     if (grid > 0x7fffffffull) return fail(BURNEXT_UNSUPPORTED, "expert GEMM grid too large");
     ProfScope ps(L, s, up ? kKGateUp : kKDown);
     st = check_launch(launch_gemm(g, up != 0, (uint32_t)grid, s), up ? "gate_up GEMM launch" : "down GEMM launch");
+    if (st != BURNEXT_OK) return st;
+  }
+  return BURNEXT_OK;
+}
+
+// The expert projections as tiles (after router and top-k): dispatch with the token-tile
+// prefix, gate_up (SwiGLU rows, f32), down (slot rows, f32).
+burnext_status run_tile_experts(burnext_moe_layer *L, bool xn_bf16, uint64_t n, const WsPtrs &p, hipStream_t s) {
+  const TileShape ts = tile_shape(n);
+  burnext_status st = run_dispatch(L, n, p.topk_idx, p.seg_off, p.perm, p.pos_of, p.active, p.num_active, p.exrec, p.dcnt,
+                                   s, p.tile_off, ts.tok);
+  if (st != BURNEXT_OK) return st;
+  const uint64_t nk = n * L->K;
+  const uint64_t max_tiles = nk / ts.tok + std::min<uint64_t>(L->E, nk);
+  const int nt = xn_bf16 ? 1 : 2;
+  for (int up = 1; up >= 0; --up) {
+    const TiledMx &t = up ? L->w1 : L->w2;
+    TileArgs g{};
+    g.wb = t.blocks;
+    g.ws = t.gscales;
+    g.wb_estride = t.blocks_per_expert;
+    g.ws_estride = t.gscales_per_expert;
+    g.bias = up ? L->b1 : L->b2;
+    g.bias_estride = t.rows_p;
+    g.nrt = t.nrt;
+    g.nb = t.nb;
+    g.kt = t.cols;
+    g.out_rows = up ? L->F : L->D;
+    g.nrb = (t.nrt + 4u * ts.row_tiles - 1u) / (4u * ts.row_tiles);
+    g.seg_off = p.seg_off;
+    g.tile_off = p.tile_off;
+    g.perm = p.perm;
+    g.E = L->E;
+    g.topk = L->K;
+    g.brows = up ? p.xn : (const void *)p.act;
+    g.bstride = up ? L->Dp : L->Fp;
+    g.out = up ? p.act : p.ypart;
+    g.out_stride = up ? L->Fp : L->Dp;
+    g.alpha = L->alpha;
+    g.limit = L->limit;
+    const uint64_t grid = align_up((uint64_t)g.nrb * max_tiles, 8);
+    if (grid > 0x7fffffffull) return fail(BURNEXT_UNSUPPORTED, "expert tile grid too large");
+    ProfScope ps(L, s, up ? kKGateUp : kKDown);
+    st = check_launch(launch_tile(g, ts, nt, up != 0, xn_bf16, (uint32_t)grid, s), up ? "gate_up tile launch" : "down tile launch");
     if (st != BURNEXT_OK) return st;
   }
   return BURNEXT_OK;
@@ -917,7 +987,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
   if (st != BURNEXT_OK) return st;
   const WsPtrs p = ws_ptrs(*L, w, workspace);
   const bool norm = (flags & BURNEXT_APPLY_RMSNORM) != 0;
-  if (w.gemm && xb) {
+  if (use_mx_gemm(*L, n, xb)) {
     st = forward_gemm(L, x, xb, n, norm, p, s);
     if (st != BURNEXT_OK) return st;
     return combine(L, x, y, xb, n, flags, p, s, 1, true);  // bf16 slot rows from the down GEMM
@@ -947,8 +1017,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     if (!route1) st = run_small_route(L, n, p, p.logits, p.topk_idx, p.topk_w, s);
   } else if (st == BURNEXT_OK) {
     st = run_topk(L, n, p.logits, p.topk_idx, p.topk_w, s);
-    if (st == BURNEXT_OK)
-      st = run_dispatch(L, n, p.topk_idx, p.seg_off, p.perm, p.pos_of, p.active, p.num_active, p.exrec, p.dcnt, s);
+    if (st == BURNEXT_OK) st = run_tile_experts(L, xnb, n, p, s);
   }
   if (st != BURNEXT_OK) return st;
 
@@ -1000,7 +1069,8 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     ProfScope ps(L, s, gate_up ? kKGateUp : kKDown);
     return check_launch(launch_gemv(g, nt, gate_up, xnb, cf.grid, s), gate_up ? "gate_up launch" : "down launch");
   };
-  st = gemv(true);
+  const bool tiles = n > kSmallRouteMaxTokens;  // the expert projections have run
+  if (!tiles) st = gemv(true);
   if (st != BURNEXT_OK) return st;
   // a single token routed in gate_up, down in kDownSplitFew parts and no fused norm: the down
   // projection and the combine in one launch (down_combine1_kernel, the same arithmetic)
@@ -1030,7 +1100,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     st = check_launch(launch_down_combine1(d, nt, xb, s), "down + combine launch");
     return st == BURNEXT_OK ? ok() : st;
   }
-  st = gemv(false);
+  if (!tiles) st = gemv(false);
   if (st != BURNEXT_OK) return st;
 
   // the fused RmsNorm of y: f32 rows of at most 4096 values (combine_norm_kernel)
@@ -1136,6 +1206,7 @@ burnext_status burnext_moe_layer_create(const burnext_moe_config *cfg, const bur
     std::call_once(once, [] {
       cfg_err = configure_kernels();
       if (cfg_err == hipSuccess) cfg_err = configure_gemm_kernels();
+      if (cfg_err == hipSuccess) cfg_err = configure_tile_kernels();
       if (cfg_err == hipSuccess) cfg_err = configure_fused_kernels();
     });
     if (cfg_err != hipSuccess) return fail(BURNEXT_DEVICE_ERROR, std::string("kernel configuration failed: ") + hipGetErrorString(cfg_err));
