@@ -11,8 +11,8 @@
 // router_small      decode-sized router (n <= 16): one wave per (expert, token pair), also
 //                   writes the normalised token rows for the expert GEMV
 // small_route       top-k/softmax/dispatch of a decode-sized batch by one workgroup
-// expert_gemv       MXFP4 x bf16 projection on MFMA 16x16x32 bf16, e2m1+e8m0 dequantised in
-//                   registers; gate_up staging applies the RmsNorm and the epilogue fuses bias +
+// expert_gemv       single-token MXFP4 x bf16 projection on MFMA 16x16x32 bf16, e2m1+e8m0 dequantised in
+//                   registers (more tokens: tile_gemm.hip, gemm.hip); gate_up staging applies the RmsNorm and the epilogue fuses bias +
 //                   clamped SwiGLU
 //                   replaces w1_swiglu_dense_kernel / w2_scatter_dense_kernel (src/quant/gpu.rs:89-192)
 // combine_kernel    y = x + sum_p w_p * (down_p + b2), deterministic slot order
@@ -1441,9 +1441,9 @@ __device__ __forceinline__ bool gemv_share(uint32_t g, uint32_t G, uint32_t na, 
   return cnt > 0u;
 }
 
+// Single-token batches that touch few experts (more tokens or experts: tile_gemm.hip).
 // Work split.  Grid of G workgroups (as many as stay resident); workgroup g owns the units
-// gemv_share gives it (decode-sized batches) or a strided share (units part + wpe * i of slot
-// g / wpe, larger batches), wave w every 4th of them from its w-th.  A unit is a row tile or (down with
+// gemv_share gives it, wave w every 4th of them from its w-th.  A unit is a row tile or (down with
 // ksplit) one of ksplit fixed K-parts of a row tile (unit u: part u / nrt of row tile u mod nrt).
 // gate_up in kGateUpSplit K-parts: the workgroup's units are row tiles and wave w takes K-part w of
 // every one of them; at each tile's end the parts meet in LDS (one barrier), wave 0 sums them in
@@ -1490,20 +1490,9 @@ __global__ __launch_bounds__(kGemvThreads) __attribute__((amdgpu_waves_per_eu(3)
     for (uint32_t i = threadIdx.x; i < nv; i += blockDim.x) dst[i] = src[i];
   }
   // this workgroup's units: lo + us * i, i < ntw (workgroup-uniform return when it has none)
-  uint32_t ai = 0, lo = 0, ntw = 0, us = 1;
-  if (a.weighted) {
-    if (!gemv_share<GATE_UP>(blockIdx.x, gridDim.x, na, nunits, a.num_cus, ai, lo, ntw)) return;
-  } else {
-    // strided: workgroup g = ai * wpe + part owns units part, part + wpe, ... of slot ai, so an
-    // expert's workgroups sweep its weights together (few pages hot at a time)
-    if (na == 0u) return;
-    const uint32_t wpe = max(1u, min(gridDim.x / na, nunits));
-    ai = blockIdx.x / wpe;
-    if (ai >= na) return;
-    lo = blockIdx.x - ai * wpe;
-    us = wpe;
-    ntw = (nunits - lo + wpe - 1u) / wpe;
-  }
+  uint32_t ai = 0, lo = 0, ntw = 0;
+  constexpr uint32_t us = 1;
+  if (!gemv_share<GATE_UP>(blockIdx.x, gridDim.x, na, nunits, a.num_cus, ai, lo, ntw)) return;
   __syncthreads();
   const int32_t *rec0 = (const int32_t *)smem + ai * kRecWords;  // valid until the first staging
   if (threadIdx.x < kRecWords) rec_l[threadIdx.x] = rec0[threadIdx.x];
@@ -2249,23 +2238,10 @@ hipError_t configure_kernels() {
   BX_ATTR((router_rows_kernel<uint16_t, uint16_t, 2>));
   BX_ATTR((router_rows_kernel<uint16_t, uint16_t, 4>));
   BX_ATTR(dispatch_kernel);
-  BX_ATTR((expert_gemv_kernel<1, true, uint16_t, 1, false>));
-  BX_ATTR((expert_gemv_kernel<1, true, float, 1, false>));
   BX_ATTR((expert_gemv_kernel<1, true, uint16_t, kGateUpSplit, false>));
-  BX_ATTR((expert_gemv_kernel<1, true, float, kGateUpSplit, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, 1, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, kDownSplit, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, kDownSplitFew, false>));
-  BX_ATTR((expert_gemv_kernel<2, true, uint16_t, 1, false>));
-  BX_ATTR((expert_gemv_kernel<2, true, float, 1, false>));
-  BX_ATTR((expert_gemv_kernel<2, true, uint16_t, kGateUpSplit, false>));
-  BX_ATTR((expert_gemv_kernel<2, true, float, kGateUpSplit, false>));
-  BX_ATTR((expert_gemv_kernel<2, false, float, 1, false>));
-  BX_ATTR((expert_gemv_kernel<2, false, float, kDownSplit, false>));
-  BX_ATTR((expert_gemv_kernel<2, false, float, kDownSplitFew, false>));
-  BX_ATTR((expert_gemv_kernel<2, true, uint16_t, 1, true>));
-  BX_ATTR((expert_gemv_kernel<2, true, float, 1, true>));
-  BX_ATTR((expert_gemv_kernel<2, true, uint16_t, kGateUpSplit, true>));
   BX_ATTR((expert_gemv_kernel<2, true, float, kGateUpSplit, true>));
   BX_ATTR((expert_gemv_kernel<2, false, float, 1, true>));
   BX_ATTR((expert_gemv_kernel<2, false, float, kDownSplit, true>));
@@ -2394,25 +2370,13 @@ hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int NT, bool PK>
-static void launch_gemv_t(const GemvArgs &a, bool gate_up, bool x_bf16, dim3 g, size_t lds, hipStream_t s) {
+template <int NT, typename XT, bool PK>
+static hipError_t launch_gemv_t(const GemvArgs &a, bool gate_up, dim3 g, size_t lds, hipStream_t s) {
   const dim3 block(kGemvThreads);
-  const bool split = !gate_up && a.ksplit > 1u;
-  const bool usplit = gate_up && a.ksplit > 1u;
-  if (split && a.ksplit == kDownSplitFew)
-    (void)launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplitFew, PK>, g, block, lds, s, a);
-  else if (split)
-    (void)launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplit, PK>, g, block, lds, s, a);
-  else if (!gate_up)
-    (void)launch_kernel(expert_gemv_kernel<NT, false, float, 1, PK>, g, block, lds, s, a);
-  else if (usplit && x_bf16)
-    (void)launch_kernel(expert_gemv_kernel<NT, true, uint16_t, kGateUpSplit, PK>, g, block, lds, s, a);
-  else if (usplit)
-    (void)launch_kernel(expert_gemv_kernel<NT, true, float, kGateUpSplit, PK>, g, block, lds, s, a);
-  else if (x_bf16)
-    (void)launch_kernel(expert_gemv_kernel<NT, true, uint16_t, 1, PK>, g, block, lds, s, a);
-  else
-    (void)launch_kernel(expert_gemv_kernel<NT, true, float, 1, PK>, g, block, lds, s, a);
+  if (gate_up) return launch_kernel(expert_gemv_kernel<NT, true, XT, kGateUpSplit, PK>, g, block, lds, s, a);
+  if (a.ksplit == kDownSplitFew) return launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplitFew, PK>, g, block, lds, s, a);
+  if (a.ksplit == kDownSplit) return launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplit, PK>, g, block, lds, s, a);
+  return launch_kernel(expert_gemv_kernel<NT, false, float, 1, PK>, g, block, lds, s, a);
 }
 
 hipError_t launch_gemv(const GemvArgs &a, int nt, bool gate_up, bool x_bf16, uint32_t grid, hipStream_t s) {
@@ -2424,16 +2388,11 @@ hipError_t launch_gemv(const GemvArgs &a, int nt, bool gate_up, bool x_bf16, uin
     return hipErrorInvalidValue;
   const size_t lds = gemv_launch_lds_bytes(nt, a.mt_max, a.nb, a.nrec, gate_up && a.ksplit > 1u);
   if (!gate_up && a.ksplit > 1u && a.ksplit != kDownSplit && a.ksplit != kDownSplitFew) return hipErrorInvalidValue;
-  if (gate_up && a.ksplit > 1u && a.ksplit != kGateUpSplit) return hipErrorInvalidValue;
-  if (nt == 1)
-    launch_gemv_t<1, false>(a, gate_up, x_bf16, g, lds, s);
-  else if (nt == 2 && 2u * a.mt_max <= 16u)  // both terms in one MFMA's columns
-    launch_gemv_t<2, true>(a, gate_up, x_bf16, g, lds, s);
-  else if (nt == 2)
-    launch_gemv_t<2, false>(a, gate_up, x_bf16, g, lds, s);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (gate_up && a.ksplit != kGateUpSplit) return hipErrorInvalidValue;
+  if (nt == 1 && (x_bf16 || !gate_up)) return launch_gemv_t<1, uint16_t, false>(a, gate_up, g, lds, s);
+  if (nt == 2 && (!x_bf16 || !gate_up) && 2u * a.mt_max <= 16u)  // both terms in one MFMA's columns
+    return launch_gemv_t<2, float, true>(a, gate_up, g, lds, s);
+  return hipErrorInvalidValue;
 }
 
 // Combine of the grouped-GEMM path (bf16 x, y and slot rows, D % 8 == 0, 16-byte aligned x and

@@ -106,7 +106,6 @@ struct GemvArgs {
   const int32_t *exrec;   // [E, kRecWords] per-active-expert records
   uint32_t nrec;          // records loaded: min(E, n * topk), every slot that can be active
   uint32_t num_cus;       // CUs of the device (dispatch rounds of the grid, see gemv_share)
-  uint32_t weighted;      // 1: gemv_share's contiguous round-weighted shares; 0: strided shares
   uint32_t topk;
   // B operand rows: gate_up xn [n, Kp] (x dtype), down act [n*k, Kp] f32 (segment order)
   const void *brows;
@@ -224,7 +223,7 @@ struct GemmArgs {
 struct TileShape {
   uint32_t row_tiles, tok;  // 16-row tiles per wave, tokens
 };
-constexpr TileShape kTileLarge = {4, 64}, kTileSmall = {2, 32};
+constexpr TileShape kTileLarge = {4, 64}, kTileSmall = {2, 32}, kTileDecode = {2, 16};
 struct TileArgs {
   const uint8_t *wb, *ws;  // tiled MXFP4 codes; scales in the GEMM's copy (as GemmArgs)
   uint64_t wb_estride, ws_estride;
@@ -233,6 +232,9 @@ struct TileArgs {
   uint32_t nrt, nb, kt, out_rows;  // out_rows: gate_up F features, down D rows
   uint32_t nrb;            // 64 row_tiles-row blocks per expert
   const int32_t *seg_off, *tile_off, *perm;
+  // t.tok == 16 (decode sizes): one tile per active expert, in tile_off's place; nperm entries in perm
+  const int32_t *active, *num_active;
+  uint32_t nperm;
   uint32_t E, topk;
   const void *brows;       // gate_up xn [n, bstride] (x dtype), down act [n*k, bstride] f32 (segment order)
   uint32_t bstride;

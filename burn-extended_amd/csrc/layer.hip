@@ -287,46 +287,30 @@ bool check_desc(const burnext_mxfp4_desc *d, uint64_t E, uint64_t rows, uint64_t
   return true;
 }
 
-// Expert GEMV launch shape for n tokens: token rows staged per pass and the persistent grid (as
+// Expert GEMV launch shape (single-token batches, one token row staged): the persistent grid (as
 // many workgroups as stay resident: LDS-limited, at most 4 per CU, at least one per possible
 // active expert; the kernel splits it among the active experts, gemv_share).
 struct GemvCfg {
-  uint32_t mt, grid, nrec;
+  uint32_t grid, nrec;
 };
 
-bool gate_up_split(const burnext_moe_layer &L, uint64_t n);
-
-GemvCfg gemv_cfg(const burnext_moe_layer &L, uint64_t n, int nt, bool gate_up) {
+GemvCfg gemv_cfg(const burnext_moe_layer &L, int nt, bool gate_up) {
   const TiledMx &t = gate_up ? L.w1 : L.w2;
   GemvCfg c{};
-  const size_t per_tok = gemv_lds_bytes(nt, 1, t.nb);
-  // LDS rows reserved for one token pass (a segment with more tokens takes another pass over its
-  // expert's weights): 8 at decode sizes and whenever routing leaves at most 4 tokens per expert on
-  // average (3 workgroups per CU at D = 2880), else the most that still lets 2 workgroups share a
-  // CU (14 at D = 2880), at most 16.  Memory parallelism beats the extra passes (measured, per
-  // step: 120B T = 64 478 -> 373 us with 8 instead of 16; 20B T = 64 / 128 / 200 282 / 292 / 410
-  // -> 192 / 243 / 335 us with 14 instead of 16).
-  const uint64_t max_active = std::min<uint64_t>(L.E, n * L.K);
-  c.nrec = (uint32_t)max_active;
-  const bool small_segments = n <= 16 || n * L.K <= 4ull * L.E;
-  // two-term (f32) activations at decode sizes: 4 rows per pass keep 3 workgroups per CU (8 rows
-  // would leave one; segments beyond 4 tokens are rare there and take a second pass)
-  uint32_t mt = (nt >= 2 && n <= 16) ? 4 : 8;
-  if (!small_segments)
-    for (mt = 16; mt > 8 && gemv_total_lds_bytes(nt, mt, t.nb, c.nrec) > 80 * 1024; --mt) {
-    }
-  mt = (uint32_t)std::min<uint64_t>(mt, n);
-  c.mt = (uint32_t)std::min<size_t>(mt, std::max<size_t>(1, (96 * 1024) / per_tok));
-  const size_t lds = gemv_launch_lds_bytes(nt, c.mt, t.nb, c.nrec, gate_up && gate_up_split(L, n));
+  c.nrec = std::min(L.E, L.K);
+  const size_t lds = gemv_launch_lds_bytes(nt, 1, t.nb, c.nrec, gate_up);
   const uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(4, (160 * 1024) / std::max<size_t>(lds, 1)));
-  c.grid = (uint32_t)std::max<uint64_t>(max_active, std::min<uint64_t>((uint64_t)L.num_cus * per_cu, max_active * t.nrt));
+  c.grid = (uint32_t)std::max<uint64_t>(c.nrec, std::min<uint64_t>((uint64_t)L.num_cus * per_cu, (uint64_t)c.nrec * t.nrt));
   return c;
 }
 
-// Decode-sized batches that touch so few experts that their gate_up row tiles are fewer than 8 per
-// CU (2/3 of a tile per wave) split every tile's K range in kGateUpSplit parts, one per wave of a
-// workgroup: a wave then streams 6 instead of 23 K-groups at D = 2880 (120B T = 1: 4 experts, 1440
-// row tiles for 3072 waves), and the workgroup sums the parts before the SwiGLU.
+// Batches that touch so few experts that their gate_up row tiles are fewer than 8 per CU (2/3 of a
+// tile per wave) can split every tile's K range in kGateUpSplit parts, one per wave of a workgroup: a
+// wave then streams 6 instead of 23 K-groups at D = 2880 (120B T = 1: 4 experts, 1440 row tiles for
+// 3072 waves), and the workgroup sums the parts before the SwiGLU.  Single tokens run so; larger
+// decode batches run as tiles, whatever they touch (measured, tiles against split GEMVs per step:
+// 8 tokens on 2 experts of D = F = 2880 35.2 / 42.8 us, 16 on 8 of 1024 26.0 / 31.5, 2 on 8 of 1024
+// 22.5 / 23.4-25.1), but the workspace is sized for both.
 bool gate_up_split(const burnext_moe_layer &L, uint64_t n) {
   return n <= kSmallRouteMaxTokens && std::min<uint64_t>(L.E, n * L.K) * L.w1.nrt < 8ull * (uint64_t)L.num_cus &&
          (L.w1.nb + 3u) / 4u >= kGateUpSplit;
@@ -347,15 +331,18 @@ inline bool gemm_regions(const burnext_moe_layer &L, uint64_t n) {
   return n >= kGemmMinTokens && n * L.K >= kGemmMinPerExpert * L.E;
 }
 
-// The expert projections by batch size: up to kSmallRouteMaxTokens tokens the expert GEMVs; beyond, as
-// tiles on bf16 MFMA (tile_gemm.hip: the GEMV's operands and precision), except bf16 batches of
+// The expert projections by batch size: a single token that touches few experts (gate_up_split) by
+// the expert GEMVs; all others as tiles on bf16 MFMA (tile_gemm.hip: the GEMV's operands and
+// precision), except bf16 batches of
 // kMxMinTokens tokens and kMxMinPerExpert routed tokens per expert, which run the grouped GEMM on the
 // block-scaled MFMA (its two activation terms carry about 2^-6 relative precision: bf16 rows only).
 // Tiles against the grouped GEMM per step, D = F = 2880, k = 4, bf16: E = 32 109 / 134 us at 64 tokens,
 // 125 / 135 at 128, 129 / 136 at 160, 141 / 139 at 200, 162 / 141 at 256; E = 128 322 / 384 at 128, 358 / 398
 // at 200, 400 / 415 at 300, 428 / 428 at 400, 448 / 439 at 512.  Against GEMV passes of 8 .. 14 token rows:
 // E = 32 bf16 98 / 107 us at 17 tokens, 101 / 113 at 45, 108 / 130 at 63, f32 115 / 133 at 17 and 340 / 1085 at
-// 523; E = 128 bf16 278 / 308 at 64, 310 / 376 at 100.
+// 523; E = 128 bf16 278 / 308 at 64, 310 / 376 at 100.  Decode sizes, tiles of 16 tokens x 128 rows against
+// GEMV passes of 8 (bf16) and 4 (f32) rows in K-halves: E = 32 bf16 39 / 50 us at 2 tokens, 53 / 62 at 4,
+// 67 / 74 at 8, 87 / 95 at 16, f32 46 / 52 at 2, 71 / 73 at 8, 92 / 113 at 16; 64-row tiles 38 / 54 / 71 / 92 (bf16).
 constexpr uint64_t kMxMinTokens = 192;
 constexpr uint64_t kMxMinPerExpert = 12;
 inline bool use_mx_gemm(const burnext_moe_layer &L, uint64_t n, bool xb) {
@@ -363,12 +350,15 @@ inline bool use_mx_gemm(const burnext_moe_layer &L, uint64_t n, bool xb) {
 }
 static_assert(kMxMinTokens >= kGemmMinTokens && kMxMinPerExpert >= kGemmMinPerExpert, "the GEMM path has its regions");
 
-// Tiles of 32 tokens x 128 rows up to 224 tokens (four workgroups a CU, weights streamed past the
+// Tiles of 16 tokens x 128 rows at decode sizes (an expert has at most 16 tokens there, and its one
+// tile needs no search), of 32 tokens x 128 rows up to 224 tokens (four workgroups a CU, weights streamed past the
 // caches), of 64 x 256 beyond (half the operand reads and weight conversions per product).  32 x 128
 // against 64 x 256 per step: E = 32 bf16 125 / 133 us at 128 tokens, 141 / 151 at 200, 181 / 162 at 256, f32
 // 170 / 187 at 200, 215 / 204 at 256; E = 128 bf16 278 / 302 at 64, 358 / 363 at 200, 406 / 400 at 300.
 constexpr uint64_t kTileSmallMaxTokens = 224;
-inline TileShape tile_shape(uint64_t n) { return n <= kTileSmallMaxTokens ? kTileSmall : kTileLarge; }
+inline TileShape tile_shape(uint64_t n) {
+  return n <= kSmallRouteMaxTokens ? kTileDecode : n <= kTileSmallMaxTokens ? kTileSmall : kTileLarge;
+}
 
 // Codes per row of the GEMM's activation rows over K = cols of a tiled projection (whole 128-wide
 // K-groups): the hi term's bytes; the lo term takes half as many.
@@ -864,11 +854,14 @@ burnext_status forward_gemm(burnext_moe_layer *L, const void *x, bool xb, uint64
 // prefix, gate_up (SwiGLU rows, f32), down (slot rows, f32).
 burnext_status run_tile_experts(burnext_moe_layer *L, bool xn_bf16, uint64_t n, const WsPtrs &p, hipStream_t s) {
   const TileShape ts = tile_shape(n);
-  burnext_status st = run_dispatch(L, n, p.topk_idx, p.seg_off, p.perm, p.pos_of, p.active, p.num_active, p.exrec, p.dcnt,
-                                   s, p.tile_off, ts.tok);
+  const bool one_tile = n <= kSmallRouteMaxTokens;  // dispatched by the routing kernel
+  burnext_status st = BURNEXT_OK;
+  if (!one_tile)
+    st = run_dispatch(L, n, p.topk_idx, p.seg_off, p.perm, p.pos_of, p.active, p.num_active, p.exrec, p.dcnt, s,
+                      p.tile_off, ts.tok);
   if (st != BURNEXT_OK) return st;
   const uint64_t nk = n * L->K;
-  const uint64_t max_tiles = nk / ts.tok + std::min<uint64_t>(L->E, nk);
+  const uint64_t max_tiles = one_tile ? std::min<uint64_t>(L->E, nk) : nk / ts.tok + std::min<uint64_t>(L->E, nk);
   const int nt = xn_bf16 ? 1 : 2;
   for (int up = 1; up >= 0; --up) {
     const TiledMx &t = up ? L->w1 : L->w2;
@@ -886,6 +879,9 @@ burnext_status run_tile_experts(burnext_moe_layer *L, bool xn_bf16, uint64_t n, 
     g.nrb = (t.nrt + 4u * ts.row_tiles - 1u) / (4u * ts.row_tiles);
     g.seg_off = p.seg_off;
     g.tile_off = p.tile_off;
+    g.active = p.active;
+    g.num_active = p.num_active;
+    g.nperm = (uint32_t)std::min<uint64_t>(nk, 1u << 30);
     g.perm = p.perm;
     g.E = L->E;
     g.topk = L->K;
@@ -1000,25 +996,20 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
   const int nt = xnb ? 1 : 2;
   FusedGeom fg{};
   const bool fused_experts = (flags & BURNEXT_FUSED_EXPERTS) && use_fused(*L, n, nt, pn != nullptr, fg);
-  // a single token routes inside the gate_up launch (route_one_token: no routing launch)
-  const bool route1 = n == 1 && !fused_experts && L->E <= kMaxExperts && L->K <= kMaxTopK && L->K <= L->E;
-  const GemvCfg cfg_up = gemv_cfg(*L, n, nt, true), cfg_dn = gemv_cfg(*L, n, nt, false);
-  // down projection of decode-sized batches: every row tile's K range in ksplit fixed parts of
-  // whole K-groups (separate work units, so the units are a fraction of a tile each and spread
-  // evenly over the waves; measured slower from 64 tokens on)
-  const bool up_split = gate_up_split(*L, n);
-  // (few touched experts: kDownSplitFew parts, as many as the workspace holds for those batches)
-  const uint32_t ksplit = (up_split && (L->w2.nb + 3u) / 4u >= kDownSplitFew) ? kDownSplitFew
-                        : (n <= kSmallRouteMaxTokens && (L->w2.nb + 3u) / 4u >= kDownSplit) ? kDownSplit : 1u;
+  // a single token that touches few experts runs the expert GEMVs and routes inside the gate_up
+  // launch (route_one_token: no routing launch); other batches run as tiles
+  const bool route1 = n == 1 && !fused_experts && gate_up_split(*L, n);
+  // its down row tiles' K range in fixed parts of whole K-groups (separate work units), as many as
+  // the workspace holds
+  const uint32_t nkg2 = (L->w2.nb + 3u) / 4u;
+  const uint32_t ksplit = !route1 ? 1u : nkg2 >= kDownSplitFew ? kDownSplitFew : nkg2 >= kDownSplit ? kDownSplit : 1u;
   st = pa             ? run_router_front(L, *pa, n, norm, p.rms, p.logits, p.xn, xnb, s)
        : small_router ? run_router_small(L, x, xb, n, norm, p.rms, p.logits, p.xn, xnb && !xb, s)
                       : run_router(L, x, xb, n, norm, p.rms, p.logits, p.xn, s, nullptr, xnb && !xb);
-  if (st == BURNEXT_OK && n <= kSmallRouteMaxTokens) {
-    if (!route1) st = run_small_route(L, n, p, p.logits, p.topk_idx, p.topk_w, s);
-  } else if (st == BURNEXT_OK) {
-    st = run_topk(L, n, p.logits, p.topk_idx, p.topk_w, s);
-    if (st == BURNEXT_OK) st = run_tile_experts(L, xnb, n, p, s);
-  }
+  if (st == BURNEXT_OK && !route1)
+    st = n <= kSmallRouteMaxTokens ? run_small_route(L, n, p, p.logits, p.topk_idx, p.topk_w, s)
+                                   : run_topk(L, n, p.logits, p.topk_idx, p.topk_w, s);
+  if (st == BURNEXT_OK && !route1 && !fused_experts) st = run_tile_experts(L, xnb, n, p, s);
   if (st != BURNEXT_OK) return st;
 
   if (fused_experts) {
@@ -1028,7 +1019,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
   }
 
   auto gemv = [&](bool gate_up) -> burnext_status {
-    const GemvCfg &cf = gate_up ? cfg_up : cfg_dn;
+    const GemvCfg cf = gemv_cfg(*L, nt, gate_up);
     const TiledMx &t = gate_up ? L->w1 : L->w2;
     GemvArgs g{};
     g.wb = t.blocks;
@@ -1041,7 +1032,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     g.nb = t.nb;
     g.kt = t.cols;
     g.out_rows = gate_up ? L->F : L->D;
-    g.mt_max = cf.mt;
+    g.mt_max = 1;
     g.seg_off = p.seg_off;
     g.active = p.active;
     g.num_active = p.num_active;
@@ -1055,13 +1046,12 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     g.limit = L->limit;
     g.nrec = cf.nrec;
     g.num_cus = (uint32_t)L->num_cus;
-    g.weighted = n <= kSmallRouteMaxTokens ? 1u : 0u;  // measured: strided shares faster from 64 tokens on
     if (!gate_up && ksplit > 1u) {
       g.ksplit = ksplit;
       g.out_half = n * L->K * L->Dp;
     }
-    if (gate_up && up_split) g.ksplit = kGateUpSplit;  // K-parts on the waves of a workgroup, summed there
-    if (gate_up && route1) {
+    if (gate_up) g.ksplit = kGateUpSplit;  // K-parts on the waves of a workgroup, summed there
+    if (gate_up) {
       g.route1_lg = p.logits;
       g.route1_E = L->E;
       g.rout = RouteOut{p.topk_idx, p.topk_w, p.seg_off, p.perm, p.pos_of, p.active, p.num_active, p.exrec};
@@ -1069,8 +1059,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     ProfScope ps(L, s, gate_up ? kKGateUp : kKDown);
     return check_launch(launch_gemv(g, nt, gate_up, xnb, cf.grid, s), gate_up ? "gate_up launch" : "down launch");
   };
-  const bool tiles = n > kSmallRouteMaxTokens;  // the expert projections have run
-  if (!tiles) st = gemv(true);
+  if (route1) st = gemv(true);
   if (st != BURNEXT_OK) return st;
   // a single token routed in gate_up, down in kDownSplitFew parts and no fused norm: the down
   // projection and the combine in one launch (down_combine1_kernel, the same arithmetic)
@@ -1100,7 +1089,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
     st = check_launch(launch_down_combine1(d, nt, xb, s), "down + combine launch");
     return st == BURNEXT_OK ? ok() : st;
   }
-  if (!tiles) st = gemv(false);
+  if (route1) st = gemv(false);
   if (st != BURNEXT_OK) return st;
 
   // the fused RmsNorm of y: f32 rows of at most 4096 values (combine_norm_kernel)

@@ -1,10 +1,11 @@
 // tile_gemm.hip -- grouped expert GEMM on bf16 MFMA with MXFP4 weights dequantised in registers: the
-// expert projections of f32 batches (and of bf16 batches too small for gemm.hip) beyond decode sizes.
+// expert projections of every f32 batch, and of the bf16 batches too small for gemm.hip, but the single
+// tokens that run the expert GEMV (kernels.hip).
 //
 // replaces w1_swiglu_dense_kernel / w2_scatter_dense_kernel (src/quant/gpu.rs:89-192) for those
 // batches (the reference runs them per 256-token tile and per used expert, src/moe/mod.rs:262-404).
 //
-// Same operands and roundings as the expert GEMV (kernels.hip): A = exact bf16 of code x scale,
+// Same operands and roundings as the expert GEMV: A = exact bf16 of code x scale,
 // B = the activation row as NT bf16 terms (bf16 rows: themselves; f32 rows: hi + bf16 of the
 // residual, or rounded once), f32 accumulation, v_mfma_f32_16x16x32_bf16.  K order: lane group q of
 // a step s supplies K [32 q + 8 s, +8) of the 128-wide K-group for both operands, which is the
@@ -17,7 +18,11 @@
 // bound by the matrix cores: 523 tokens 793 + 423 -> 182 + 117 us, 4096 tokens 918 + 483 us (1.16
 // PFLOP/s of the two terms' products; plain bf16 MFMAs reach 1.8).  Weights are read nontemporally
 // in the 32-token shape only (gate_up 58 -> 50 us at 45 tokens: the router rows and token rows stay in
-// the caches); the 64-token shape re-reads them from L2 for the next tiles.
+// the caches); the 64-token shape re-reads them from L2 for the next tiles.  At decode sizes the
+// short items refill the CUs as they end, where the GEMV's fixed shares waited for the slowest: 8 tokens
+// 38 + 22 -> 35 + 19 us, 16 tokens in f32 64 + 33 -> 52 + 27 us, D = F = 256 with 16 tokens 14 + 13 -> 7 + 7 us
+// (every prefix and segment entry an item needs comes in one round trip, and waves whose token
+// columns are all empty skip the split).
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -92,6 +97,7 @@ struct Item {
   uint32_t rb, m0, ntok;
   int32_t *rows_l;  // LDS [TOK]: B row of each token (columns beyond the tile: its first token's)
   int32_t *slot_l;  // LDS [TOK]: down's output slot
+  const int32_t *perm_l;  // LDS (TOK 16): the batch's segment entries
   uint8_t *ring;    // LDS: [2 buffers][NT terms][TOK][256 bytes], and the epilogue's staging
 };
 
@@ -107,10 +113,11 @@ template <bool GATE_UP, typename XT, int NT, uint32_t RT, uint32_t TOK, int NTT>
 __device__ __forceinline__ void tile_body(const TileArgs &a, const Item &it) {
   constexpr uint32_t kTermBytes = term_bytes(TOK), kRows = 16u * RT * kWaves;
   using SReg = typename ScaleRegs<RT>::type;
-  // the segment entries first: their round trip runs beside the first weights'
+  // the segment entries (decode sizes: already in LDS) first: their round trip runs beside the first
+  // weights'
   int32_t slot = 0;
   const uint32_t m_own = it.m0 + (threadIdx.x < it.ntok ? threadIdx.x : 0u);
-  if (threadIdx.x < TOK) slot = a.perm[it.seg0 + (int32_t)m_own];
+  if (threadIdx.x < TOK) slot = TOK == 16u ? it.perm_l[it.seg0 + (int32_t)m_own] : a.perm[it.seg0 + (int32_t)m_own];
   const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t i16 = lane & 15u, q = lane >> 4;
   const uint32_t nkg = (a.nb + 3u) >> 2, tail = a.nb - 4u * (nkg - 1u), nkq = (nkg + 3u) >> 2, ngr = (a.nrt + 3u) >> 2;
@@ -129,7 +136,7 @@ __device__ __forceinline__ void tile_body(const TileArgs &a, const Item &it) {
     const uint32_t off = lane * 16u + ((kg + 1u == nkg && q >= tail) ? 0u : kg * 1024u);
 #pragma unroll
     for (uint32_t rt = 0; rt < RT; ++rt)
-      A[rt] = RT == 2u ? __builtin_nontemporal_load((const u32x4_t *)(arow[rt] + off)) : *(const u32x4_t *)(arow[rt] + off);
+      A[rt] = RT <= 2u ? __builtin_nontemporal_load((const u32x4_t *)(arow[rt] + off)) : *(const u32x4_t *)(arow[rt] + off);
   };
   // weights PA and B chunks PB K-groups ahead: few token columns leave registers for more
   constexpr uint32_t PA = NTT <= 2 ? 4u : 2u, PB = NTT == 1 ? 4u : NTT == 2 ? 2u : 1u;
@@ -158,13 +165,12 @@ __device__ __forceinline__ void tile_body(const TileArgs &a, const Item &it) {
   // MASK: K-group kg may be the last (zeros from kt on)
   auto stage_store = [&](uint32_t kg, uint32_t buf, BChunk<XT> (&R)[NTT], auto MASK) {
     uint8_t *st = it.ring + buf * (NT * kTermBytes);
-    if constexpr (decltype(MASK)::value) {
-      const uint32_t k = kg * 128u + 8u * ch, nv = k < a.kt ? min(8u, a.kt - k) : 0u;
-#pragma unroll
-      for (int p = 0; p < NTT; ++p) bchunk_mask(R[p], nv);
-    }
+    const uint32_t k = kg * 128u + 8u * ch, nv = k < a.kt ? min(8u, a.kt - k) : 0u;
 #pragma unroll
     for (int p = 0; p < NTT; ++p) {
+      // (wave-uniform) columns beyond the tile keep what LDS holds: their results are never stored
+      if (16u * (uint32_t)p + 4u * wv >= it.ntok) continue;
+      if constexpr (decltype(MASK)::value) bchunk_mask(R[p], nv);
       const uint32_t t = tk + 16u * (uint32_t)p;
       uint4 terms[NT];
       bchunk_terms<NT>(R[p], terms);
@@ -305,7 +311,8 @@ __device__ __forceinline__ void tile_body(const TileArgs &a, const Item &it) {
 }  // namespace
 
 size_t tile_lds_bytes(int nt, const TileShape &t) {
-  return ring_bytes(nt, t.row_tiles, t.tok) + 2 * t.tok * 4 + 64 + 2 * (kMaxExperts + 1) * 4;
+  return ring_bytes(nt, t.row_tiles, t.tok) + 2 * t.tok * 4 + 64 + 2 * (kMaxExperts + 1) * 4 +
+         (t.tok == 16u ? kSmallRouteMaxTokens * kMaxTopK * 4 : 0u);
 }
 
 // Work items (token tile of TOK routed tokens of one expert, block of 64 RT weight rows) in the
@@ -313,43 +320,57 @@ size_t tile_lds_bytes(int nt, const TileShape &t) {
 // in groups of 8 token tiles, row block by row block, so that an XCD's L2 serves the weights of a
 // group and its B rows repeatedly.
 template <bool GATE_UP, typename XT, int NT, uint32_t RT, uint32_t TOK>
-__global__ __launch_bounds__(256, RT == 2 ? 4 : 2) void expert_tile_kernel(TileArgs a) {
+__global__ __launch_bounds__(256, RT <= 2 ? 4 : 2) void expert_tile_kernel(TileArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   int32_t *rows_l = (int32_t *)(smem + ring_bytes(NT, RT, TOK));
   int32_t *slot_l = rows_l + TOK, *info_l = slot_l + TOK, *toff_l = info_l + 16, *soff_l = toff_l + kMaxExperts + 1;
+  // every prefix an item needs in one round trip; decode-sized batches (TOK 16) have one tile per
+  // active expert, listed in `active`
+  constexpr bool kOneTile = TOK == 16u;
   for (uint32_t t = threadIdx.x; t <= a.E; t += blockDim.x) {
-    toff_l[t] = a.tile_off[t];
+    toff_l[t] = !kOneTile ? a.tile_off[t] : t < a.E ? a.active[t] : *a.num_active;
     soff_l[t] = a.seg_off[t];
   }
+  int32_t *perm_l = soff_l + kMaxExperts + 1;
+  if constexpr (kOneTile)
+    for (uint32_t t = threadIdx.x; t < a.nperm; t += blockDim.x) perm_l[t] = a.perm[t];
   if (threadIdx.x == 0) info_l[0] = -1;
   __syncthreads();
   const uint32_t b = blockIdx.x, ntile = (uint32_t)toff_l[a.E], N = a.nrb * ntile, Q = (N + 7u) / 8u;
   const uint32_t item = (b & 7u) * Q + (b >> 3);
   if ((b >> 3) >= Q || item >= N) return;  // workgroup-uniform: no item
-  const uint32_t grp = item / (8u * a.nrb), r = item - grp * 8u * a.nrb, gsz = min(8u, ntile - grp * 8u);
-  const uint32_t rb = r / gsz, gt = grp * 8u + (r - rb * gsz);
-  for (uint32_t e = threadIdx.x; e < a.E; e += blockDim.x)
-    if (gt >= (uint32_t)toff_l[e] && gt < (uint32_t)toff_l[e + 1]) {
-      info_l[0] = (int32_t)e;
-      info_l[1] = (int32_t)(gt - (uint32_t)toff_l[e]);
-    }
-  __syncthreads();
+  uint32_t rb, gt;
+  if constexpr (kOneTile) {
+    gt = item / a.nrb;
+    rb = item - gt * a.nrb;
+  } else {
+    const uint32_t grp = item / (8u * a.nrb), r = item - grp * 8u * a.nrb, gsz = min(8u, ntile - grp * 8u);
+    rb = r / gsz;
+    gt = grp * 8u + (r - rb * gsz);
+    for (uint32_t e = threadIdx.x; e < a.E; e += blockDim.x)
+      if (gt >= (uint32_t)toff_l[e] && gt < (uint32_t)toff_l[e + 1]) {
+        info_l[0] = (int32_t)e;
+        info_l[1] = (int32_t)(gt - (uint32_t)toff_l[e]);
+      }
+    __syncthreads();
+  }
   Item it;
-  it.e = __builtin_amdgcn_readfirstlane(info_l[0]);
+  it.e = __builtin_amdgcn_readfirstlane(kOneTile ? toff_l[gt] : info_l[0]);
   if (it.e < 0) return;  // workgroup-uniform
   it.seg0 = __builtin_amdgcn_readfirstlane(soff_l[it.e]);
   const uint32_t M = (uint32_t)(__builtin_amdgcn_readfirstlane(soff_l[it.e + 1]) - it.seg0);
   it.rb = rb;
-  it.m0 = (uint32_t)__builtin_amdgcn_readfirstlane(info_l[1]) * TOK;
+  it.m0 = kOneTile ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(info_l[1]) * TOK;
   it.ntok = min(TOK, M - it.m0);
   it.rows_l = rows_l;
   it.slot_l = slot_l;
+  it.perm_l = perm_l;
   it.ring = smem;
   const uint32_t c16 = (it.ntok + 15u) / 16u;
-  if (c16 == 1u) return tile_body<GATE_UP, XT, NT, RT, TOK, 1>(a, it);
+  if (TOK == 16u || c16 == 1u) return tile_body<GATE_UP, XT, NT, RT, TOK, 1>(a, it);
   if constexpr (TOK == 32u) {
     return tile_body<GATE_UP, XT, NT, RT, TOK, 2>(a, it);
-  } else {
+  } else if constexpr (TOK == 64u) {
     if (c16 == 2u) return tile_body<GATE_UP, XT, NT, RT, TOK, 2>(a, it);
     if (c16 == 3u) return tile_body<GATE_UP, XT, NT, RT, TOK, 3>(a, it);
     return tile_body<GATE_UP, XT, NT, RT, TOK, 4>(a, it);
@@ -358,23 +379,26 @@ __global__ __launch_bounds__(256, RT == 2 ? 4 : 2) void expert_tile_kernel(TileA
 
 namespace {
 using TileKernel = void (*)(TileArgs);
+template <uint32_t RT, uint32_t TOK>
+TileKernel tile_kernel_of(int nt, bool gate_up, bool x_bf16) {
+  if (gate_up && nt == 1 && x_bf16) return expert_tile_kernel<true, uint16_t, 1, RT, TOK>;
+  if (gate_up && nt == 2 && !x_bf16) return expert_tile_kernel<true, float, 2, RT, TOK>;
+  if (!gate_up && nt == 1) return expert_tile_kernel<false, float, 1, RT, TOK>;
+  if (!gate_up && nt == 2) return expert_tile_kernel<false, float, 2, RT, TOK>;
+  return nullptr;
+}
 // The instantiation of a launch, null if there is none.
 TileKernel tile_kernel(int nt, bool gate_up, bool x_bf16, const TileShape &t) {
-  const bool small = t.row_tiles == 2u && t.tok == 32u;
-  if (!small && !(t.row_tiles == 4u && t.tok == 64u)) return nullptr;
-  if (gate_up && nt == 1 && x_bf16)
-    return small ? expert_tile_kernel<true, uint16_t, 1, 2, 32> : expert_tile_kernel<true, uint16_t, 1, 4, 64>;
-  if (gate_up && nt == 2 && !x_bf16)
-    return small ? expert_tile_kernel<true, float, 2, 2, 32> : expert_tile_kernel<true, float, 2, 4, 64>;
-  if (!gate_up && nt == 1) return small ? expert_tile_kernel<false, float, 1, 2, 32> : expert_tile_kernel<false, float, 1, 4, 64>;
-  if (!gate_up && nt == 2) return small ? expert_tile_kernel<false, float, 2, 2, 32> : expert_tile_kernel<false, float, 2, 4, 64>;
+  if (t.row_tiles == kTileLarge.row_tiles && t.tok == kTileLarge.tok) return tile_kernel_of<kTileLarge.row_tiles, kTileLarge.tok>(nt, gate_up, x_bf16);
+  if (t.row_tiles == kTileSmall.row_tiles && t.tok == kTileSmall.tok) return tile_kernel_of<kTileSmall.row_tiles, kTileSmall.tok>(nt, gate_up, x_bf16);
+  if (t.row_tiles == kTileDecode.row_tiles && t.tok == kTileDecode.tok) return tile_kernel_of<kTileDecode.row_tiles, kTileDecode.tok>(nt, gate_up, x_bf16);
   return nullptr;
 }
 }  // namespace
 
 hipError_t configure_tile_kernels() {
   hipError_t err = hipSuccess;
-  for (const TileShape &t : {kTileSmall, kTileLarge})
+  for (const TileShape &t : {kTileDecode, kTileSmall, kTileLarge})
     for (int nt = 1; nt <= 2; ++nt)
       for (int up = 0; up <= 1; ++up) {
         const hipError_t e = hipFuncSetAttribute((const void *)tile_kernel(nt, up != 0, nt == 1, t),
@@ -388,7 +412,8 @@ hipError_t launch_tile(const TileArgs &a, const TileShape &t, int nt, bool gate_
                        hipStream_t s) {
   const TileKernel k = tile_kernel(nt, gate_up, x_bf16, t);
   if (!k || grid == 0 || (grid & 7u) != 0 || a.nrb == 0 || a.nrt == 0 || a.nb == 0 || a.bstride % 32u != 0 ||
-      a.bstride < a.kt || a.out_stride % 4u != 0 || a.E > kMaxExperts || a.bias_estride % 16u != 0)
+      a.bstride < a.kt || a.out_stride % 4u != 0 || a.E > kMaxExperts || a.bias_estride % 16u != 0 ||
+      (t.tok == 16u && a.nperm > kSmallRouteMaxTokens * kMaxTopK))
     return hipErrorInvalidValue;
   return launch_kernel(k, dim3(grid), dim3(64 * kWaves), tile_lds_bytes(nt, t), s, a);
 }

@@ -1,5 +1,5 @@
-"""GPU: the expert projections as tiles on bf16 MFMA (batches beyond decode size off the grouped
-GEMM path) against the oracle on every row: token tiles of 1..64 rows, row blocks and K-groups with
+"""GPU: the expert projections as tiles on bf16 MFMA (all batches but single tokens on few experts and
+those of the grouped GEMM) against the oracle on every row: token tiles of 1..64 rows, row blocks and K-groups with
 remainders, one and several tiles per expert.  Bars as the other forwards': f32 rows 1e-4 (two bf16
 terms, 2^-17 per value), bf16 rows 2e-2."""
 import numpy as np
@@ -23,6 +23,14 @@ TOL = {"f32": 1e-4, "bf16": 2e-2}
     (50, 31, 6, 2, 60, "bf16", "halves", 0),           # odd F: the last value of a row segment alone
     (2880, 2880, 128, 4, 63, "bf16", "interleaved", 3),
     (2880, 2880, 32, 4, 17, "bf16", "interleaved", 3),
+    # decode sizes: one tile of up to 16 tokens per active expert
+    (256, 256, 2, 2, 16, "f32", "interleaved", 3),     # full tiles
+    (200, 100, 3, 3, 2, "bf16", "halves", 3),          # partial K-groups
+    (33, 40, 40, 32, 16, "f32", "interleaved", 3),     # the most segment entries (16 x 32)
+    (640, 1152, 256, 8, 7, "bf16", "interleaved", 1),  # the most experts
+    (50, 31, 6, 2, 11, "f32", "interleaved", 0),
+    (2880, 2880, 32, 4, 2, "f32", "interleaved", 3),
+    (1024, 2048, 64, 16, 1, "bf16", "interleaved", 3), # one token on too many experts for the GEMVs
 ])
 def test_forward_tiles_all_rows(oracle, D, F, E, K, n, dtype, layout, flags):
     from burnext_amd import moe, synth
