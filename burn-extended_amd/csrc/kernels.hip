@@ -2,8 +2,8 @@
 //
 // router_kernel     RmsNorm + router logits, parallel over token blocks x expert groups
 //                   replaces src/moe/mod.rs:109-110 (Burn RmsNorm / Linear)
-// router_rows       the same for prefill batches: one wave per few tokens, rows in registers,
-//                   also writes the two-term (MXFP8 hi + MXFP4 lo) rows of the grouped GEMM
+// router_mfma       the same for large batches on K = 1 matrix steps (the order kept), also writes the
+//                   two-term (MXFP8 hi + MXFP4 lo) rows of the grouped GEMM
 // topk_kernel       top-k + softmax over the selected logits, one wave per token
 //                   replaces src/moe/mod.rs:271-276 (topk_with_indices, max/exp/sum/div)
 // dispatch_kernel   histogram / exclusive scan / stable scatter into expert segments
@@ -322,226 +322,197 @@ __global__ __launch_bounds__(kRouterThreads) void router_kernel(RouterArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Prefill router (D % 8 == 0, D, Dp and the two-term row length <= 512 * kFrontChunks, 16-byte
-// aligned rows).  Workgroup of kRowsThreads: wave w holds tokens T (8 b + w) .. +T in registers
-// (f32, T = 2 or 4); the router rows pass through LDS as f32 in stages of kRowsExperts experts (double
-// buffered, filled by all threads, one barrier per stage), so each row is converted once per
-// workgroup and read by every wave from LDS.  LDS row layout: element 512 i + 8 l + j at
-// 512 i + 256 (j / 4) + 4 l + j % 4, so lane l's two float4 of its chunk are conflict-free.
-// Same fixed reduction order and formulas as router_kernel (lane l owns chunks c = 512 i + 8 l + j,
-// fmaf over i then j, xor butterfly; logit = dot / r + b): the logits, r and the written rows
-// equal router_kernel's bit for bit.  The two-term rows come from the registers: a 32-value
-// block is the 8-value chunks of lanes 4 b .. 4 b + 3, its maxima taken over those four lanes.
+// Router of large batches (D % 8 == 0, 16-byte aligned rows).  Workgroup (16 tokens, 16 experts) of 8
+// waves.  The fixed reduction order gives each (token, expert) 64 independent chains, chain l over the
+// chunks c = 512 i + 8 l + j (fmaf over i, then j), added by the xor butterfly.  A K = 1 matrix step
+// (v_mfma_f32_16x16x1_4b_f32: D[b] += x_b w_b^T for 4 independent 16 x 16 blocks b) is one fmaf of each of
+// 16 tokens x 16 experts x 4 chains, so the chains run on the matrix cores with the order kept: block b
+// of wave w and group g is chain l = 32 g + 4 w + b.  The butterfly: level 32 adds the two groups'
+// registers, 16 / 8 / 4 the waves' results through LDS, 2 / 1 the four blocks (addition commutes: the
+// butterfly's bits).  Each lane's x chunks are also its token's sum-of-squares chain.  Logits, r and the
+// written rows equal router_kernel's bit for bit.
+// Why: router_kernel stages 94 KB of token rows a workgroup and pays an LDS read per two products;
+// here an operand register feeds 16 products, straight from L2, and up to four workgroups share a
+// CU, so that one's round trips and row writing overlap another's products (36 KB of LDS; 32 experts
+// a workgroup, half the token reads: 37 us for 30 at E = 32, 4096 tokens).  E = 128: 1021 tokens 94 -> 23
+// us, 4096 tokens 112 -> 84; E = 32: 1024 tokens 33 -> 19, 4096 tokens 39 -> 30 (the former kernel of
+// those sizes kept 2 or 4 tokens' rows in each wave's registers).
+// Lanes past D, tokens past n and experts past E work on zeros or on a clamped row, never stored.
 // ---------------------------------------------------------------------------------------------
-constexpr int kRowsExperts = 4;    // experts per LDS stage
-constexpr uint32_t kRowsSpan = 512u * kFrontChunks;  // f32 LDS row stride
-size_t router_rows_lds_bytes() { return sizeof(float) * (2u * kRowsExperts * kRowsSpan + kMaxExperts); }
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+constexpr uint32_t kRouterTok = 16, kRouterWaves = 8;
 
-template <typename XT, typename WT, int T>  // T tokens per wave (2, or 4 for the largest batches)
-__global__ __launch_bounds__(kRowsThreads) void router_rows_kernel(RouterArgs a) {
-  constexpr int G = kRowsExperts, RC = kFrontChunks;
-  constexpr uint32_t FC = (G * kRowsSpan / 8u + kRowsThreads - 1u) / kRowsThreads;  // fill chunks per thread
-  extern __shared__ __align__(16) float wls[];  // [2][G][kRowsSpan], then rb [E]
-  float *rbl = wls + 2u * G * kRowsSpan;
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t t0 = (blockIdx.x * (kRowsThreads / 64u) + (threadIdx.x >> 6)) * (uint32_t)T;
-  const bool active = t0 < a.n;  // wave-uniform; inactive waves still fill and meet the barriers
-  const uint32_t D = a.D, E = a.E, cpr = D / 8u;  // chunks per router row
-  const XT *x = (const XT *)a.x;
-  const WT *rw = (const WT *)a.rw;
-  const uint32_t nt = active ? min((uint32_t)T, a.n - t0) : 0u;
-  const uint32_t nstage = (E + G - 1u) / G;
-
-  // stage fill: chunk f = threadIdx.x + kRowsThreads m of a stage is chunk ch = f % cpr (= 64 i + l)
-  // of the stage's expert row k = f / cpr
-  uint32_t fk[FC], fsrc[FC], fdst[FC];
+template <typename XT, typename WT>
+__global__ __launch_bounds__(64 * kRouterWaves, 4) void router_mfma_kernel(RouterArgs a) {
+  __shared__ __align__(16) float red[kRouterWaves * 1024u];  // [wave][block][lane][4]
+  __shared__ float ssl[64u * kRouterTok], rr[kRouterTok];    // [chain][token], [token]
+  const uint32_t D = a.D, E = a.E, tid = threadIdx.x;
+  const uint32_t lane = tid & 63u, w = __builtin_amdgcn_readfirstlane(tid >> 6), b = lane >> 4, m = lane & 15u;
+  const uint32_t t0 = blockIdx.x * kRouterTok, e0 = blockIdx.y * 16u, nh = min(kRouterTok, a.n - t0);
+  const XT *xr = (const XT *)a.x + (size_t)min(t0 + m, a.n - 1u) * D;
+  const WT *wr = (const WT *)a.rw + (size_t)min(e0 + m, E - 1u) * D;
+  f32x16_t acc[2];
 #pragma unroll
-  for (uint32_t m = 0; m < FC; ++m) {
-    const uint32_t f = threadIdx.x + kRowsThreads * m, k = f / cpr, ch = f - k * cpr;
-    fk[m] = k;
-    fsrc[m] = k * D + ch * 8u;
-    fdst[m] = k * kRowsSpan + (ch >> 6) * 512u + (ch & 63u) * 4u;
-  }
-  Chunk8<WT> fr[FC];
-  auto fill_load = [&](uint32_t st) {
+  for (int g = 0; g < 2; ++g)
 #pragma unroll
-    for (uint32_t m = 0; m < FC; ++m)
-      if (fk[m] < (uint32_t)G && st * G + fk[m] < E) chunk_load(fr[m], rw + (size_t)st * G * D + fsrc[m]);
+    for (int r = 0; r < 16; ++r) acc[g][r] = 0.0f;
+  float ss[2] = {0.0f, 0.0f};
+  const uint32_t c_own = 8u * (4u * w + b), steps = (D + 511u) / 512u;
+  // S steps of both groups' chunks in flight.  One copy of the step: the loop moves the registers on
+  // instead of unrolling (code that runs once per launch comes from a cold instruction cache: six
+  // copies took a 17-token launch from 15 to 26 us)
+  constexpr int S = 3;
+  Chunk8<XT> xc[S][2];
+  Chunk8<WT> wc[S][2];
+  auto load = [&](uint32_t i, int s, uint32_t g) {
+    const uint32_t c = 512u * min(i, steps - 1u) + 256u * g + c_own, off = c < D ? c : 0u;
+    chunk_load(xc[s][g], xr + off);
+    chunk_load(wc[s][g], wr + off);
   };
-  auto fill_store = [&](uint32_t st, uint32_t buf) {
 #pragma unroll
-    for (uint32_t m = 0; m < FC; ++m) {
-      if (fk[m] < (uint32_t)G && st * G + fk[m] < E) {
-        float v[8];
-        chunk_vals(fr[m], v);
-        float *d = wls + buf * G * kRowsSpan + fdst[m];
-        *(float4 *)d = make_float4(v[0], v[1], v[2], v[3]);
-        *(float4 *)(d + 256) = make_float4(v[4], v[5], v[6], v[7]);
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (uint32_t g = 0; g < 2u; ++g) load((uint32_t)s, s, g);
+#pragma unroll 1
+  for (uint32_t i = 0; i < steps; ++i) {
+#pragma unroll
+    for (uint32_t g = 0; g < 2u; ++g) {
+      float xv[8], wv[8];
+      chunk_vals(xc[0][g], xv);
+      chunk_vals(wc[0][g], wv);
+#pragma unroll
+      for (int s = 0; s + 1 < S; ++s) {
+        xc[s][g] = xc[s + 1][g];
+        wc[s][g] = wc[s + 1][g];
       }
-    }
-  };
-  fill_load(0);
-  for (uint32_t e = threadIdx.x; e < E; e += kRowsThreads) rbl[e] = a.rb[e];
-  // zeros at the chunk positions beyond D of every row (never filled): the dot loop runs over
-  // all RC chunks, and fmaf(0, 0, acc) == acc for the +0-started sums
-  for (uint32_t f = threadIdx.x; f < 2u * G * (RC * 64u - cpr); f += kRowsThreads) {
-    const uint32_t row = f / (RC * 64u - cpr), ch = cpr + (f - row * (RC * 64u - cpr));
-    float *d = wls + row * kRowsSpan + (ch >> 6) * 512u + (ch & 63u) * 4u;
-    *(float4 *)d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    *(float4 *)(d + 256) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  }
-
-  // this wave's token rows as f32 (zeros beyond D), every chunk requested before any is used: no
-  // branch around a load (a branch per chunk made the wave wait for the chunks one by one), so
-  // chunks past D or of an inactive wave read a valid chunk and are zeroed
-  float xv[T][RC][8];
-  {
-    Chunk8<XT> cx[T][RC];
+      const bool ok = 512u * i + 256u * g + c_own < D;
 #pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int i = 0; i < RC; ++i) {
-        const uint32_t c0 = min(512u * i + 8u * lane, D - 8u);
-        const uint32_t row = min(t0 + min((uint32_t)t, max(nt, 1u) - 1u), a.n - 1u);
-        chunk_load(cx[t][i], x + (size_t)row * D + c0);
+      for (int j = 0; j < 8; ++j) {
+        xv[j] = ok ? xv[j] : 0.0f;
+        wv[j] = ok ? wv[j] : 0.0f;
       }
+      load(i + (uint32_t)S, S - 1, g);
 #pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int i = 0; i < RC; ++i) {
-        const bool ok = active && 512u * i + 8u * lane < D;
-        chunk_vals(cx[t][i], xv[t][i]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) xv[t][i][j] = ok ? xv[t][i][j] : 0.0f;
-      }
-  }
-
-  // r per token
-  float r[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t) r[t] = 1.0f;
-  if (a.apply_norm) {
-    float ss[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      ss[t] = 0.0f;
-#pragma unroll
-      for (int i = 0; i < RC; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ss[t] = fmaf(xv[t][i][j], xv[t][i][j], ss[t]);
-    }
-    wave_sum_to_lane0_n<T>(ss);
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      r[t] = sqrtf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ss[t]), 0)) / (float)D + a.eps);
-      if (a.rms && lane == 0 && (uint32_t)t < nt) a.rms[t0 + t] = r[t];
-    }
-  }
-
-  // normalised rows xn = x * (1/r) * gamma (x without RmsNorm), zero padded to Dp, and their
-  // two-term form zero padded to the K-group length; written before the dot products so
-  // the stores drain meanwhile
-  if (active && (a.xn || a.xq.hi)) {
-#pragma unroll
-    for (int i = 0; i < RC; ++i) {
-      const uint32_t c0 = 512u * i + 8u * lane;
-      if (512u * i >= max(a.xn ? a.Dp : 0u, a.xq.hi ? a.xq.kq : 0u)) break;  // wave-uniform
-      float g[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) g[j] = 1.0f;
-      if (a.apply_norm && c0 < D) {
-        const float4 g0 = *(const float4 *)(a.gamma + c0), g1 = *(const float4 *)(a.gamma + c0 + 4);
-        g[0] = g0.x; g[1] = g0.y; g[2] = g0.z; g[3] = g0.w; g[4] = g1.x; g[5] = g1.y; g[6] = g1.z; g[7] = g1.w;
-      }
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const float ir = a.apply_norm ? 1.0f / r[t] : 1.0f;
-        float u[8];  // zeros beyond D: xv is zero there and gamma one
-#pragma unroll
-        for (int j = 0; j < 8; ++j) u[j] = a.apply_norm ? (xv[t][i][j] * ir) * g[j] : xv[t][i][j];
-        const size_t row = t0 + (uint32_t)t;
-        const bool tv = (uint32_t)t < nt;
-        if (a.xn && tv && c0 < a.Dp) store8((XT *)a.xn + row * a.Dp + c0, u);
-        if (a.xq.hi && 512u * i < a.xq.kq) {  // wave-uniform
-          float amax = 0.0f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(u[j]));
-          amax = fmaxf(amax, dpp_mov<0xB1>(amax));  // lanes 4 b .. 4 b + 3 hold block b
-          amax = fmaxf(amax, dpp_mov<0x4E>(amax));
-          const uint32_t sbh = mx8_scale_byte(amax);
-          const float ih = sbh ? mx8_inv_scale(sbh) : 0.0f, sh = e8m0_to_f32(sbh);
-          uint32_t ch[4];
-          float res[8], rmax = 0.0f;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            ch[k] = f32x2_to_fp8x2(u[2 * k] * ih, u[2 * k + 1] * ih);
-            res[2 * k] = u[2 * k] - fp8_to_f32<0>(ch[k]) * sh;
-            res[2 * k + 1] = u[2 * k + 1] - fp8_to_f32<1>(ch[k]) * sh;
-            rmax = fmaxf(rmax, fmaxf(fabsf(res[2 * k]), fabsf(res[2 * k + 1])));
-          }
-          rmax = fmaxf(rmax, dpp_mov<0xB1>(rmax));
-          rmax = fmaxf(rmax, dpp_mov<0x4E>(rmax));
-          const uint32_t sbl = mx4_scale_byte(rmax);
-          const float sl = mx4_divisor(sbl);
-          if (tv && c0 < a.xq.kq) {
-            uint32_t cl = 0u;
-            cl = e2m1x2<0>(cl, res[0], res[1], sl);
-            cl = e2m1x2<1>(cl, res[2], res[3], sl);
-            cl = e2m1x2<2>(cl, res[4], res[5], sl);
-            cl = e2m1x2<3>(cl, res[6], res[7], sl);
-            *(uint2 *)(a.xq.hi + row * a.xq.kq + c0) = make_uint2(ch[0] | (ch[1] << 16), ch[2] | (ch[3] << 16));
-            *(uint32_t *)(a.xq.lo + row * (a.xq.kq / 2u) + c0 / 2u) = cl;
-            if ((lane & 3u) == 0u) {
-              a.xq.shi[row * a.xq.ss + (c0 >> 5)] = (uint8_t)sbh;
-              a.xq.slo[row * a.xq.ss + (c0 >> 5)] = (uint8_t)sbl;
-            }
-          }
-        }
+      for (int j = 0; j < 8; ++j) {
+        ss[g] = fmaf(xv[j], xv[j], ss[g]);
+        acc[g] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[j], wv[j], acc[g], 0, 0, 0);
       }
     }
   }
 
-  fill_store(0, 0);
+#pragma unroll
+  for (uint32_t g = 0; g < 2u; ++g) ssl[(32u * g + 4u * w + b) * kRouterTok + m] = ss[g];
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k) {  // block k: rows (tokens) 4 (lane / 16) + r of column (expert) lane % 16
+    const f32x16_t &p = acc[0], &q = acc[1];
+    *(float4 *)(red + (w * 4u + k) * 256u + lane * 4u) =
+        make_float4(p[4 * k] + q[4 * k], p[4 * k + 1] + q[4 * k + 1], p[4 * k + 2] + q[4 * k + 2], p[4 * k + 3] + q[4 * k + 3]);
+  }
   __syncthreads();
-
-  // dot products, G experts per stage; lane q < G * T finishes (expert st * G + q / T, token q % T)
-  for (uint32_t st = 0; st < nstage; ++st) {
-    const uint32_t buf = st & 1u;
-    if (st + 1u < nstage) fill_load(st + 1u);
-    if (active) {
-      float acc[G * T];
+  if (a.apply_norm && w == kRouterWaves - 1u) {
+    // lane (b, m): chains b + 4 k of token m; levels 32 .. 4 over k, then 2 and 1 over b
+    float v[16];
 #pragma unroll
-      for (int q = 0; q < G * T; ++q) acc[q] = 0.0f;
+    for (uint32_t k = 0; k < 16u; ++k) v[k] = ssl[(b + 4u * k) * kRouterTok + m];
 #pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const float *wrow = wls + (buf * G + k) * kRowsSpan + lane * 4u;
+    for (uint32_t off = 8u; off >= 1u; off >>= 1)
 #pragma unroll
-        for (int i = 0; i < RC; ++i) {
-          const float4 w0 = *(const float4 *)(wrow + 512u * i), w1 = *(const float4 *)(wrow + 512u * i + 256u);
-          const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-          for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[k * T + t] = fmaf(xv[t][i][j], w[j], acc[k * T + t]);
-        }
-      }
-      wave_sum_to_lane0_n<G * T>(acc);
-      float v = 0.0f, rq = r[0];
-#pragma unroll
-      for (int q = 0; q < G * T; ++q) {
-        const float aq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc[q]), 0));
-        if (lane == (uint32_t)q) {
-          v = aq;
-          rq = r[q % T];
-        }
-      }
-      const uint32_t e = st * G + lane / T, t = lane % T;
-      if (lane < (uint32_t)(G * T) && e < E && t < nt)
-        a.logits[(size_t)(t0 + t) * E + e] = (a.apply_norm ? v / rq : v) + rbl[e];
+      for (uint32_t k = 0; k < off; ++k) v[k] = v[k] + v[k + off];
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[0]), false, false);
+    const float s2 = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    const auto p1 = __builtin_amdgcn_permlane16_swap(__float_as_uint(s2), __float_as_uint(s2), false, false);
+    const float s1 = __uint_as_float(p1[0]) + __uint_as_float(p1[1]);
+    const float r = sqrtf(s1 / (float)D + a.eps);
+    if (lane < kRouterTok) {
+      rr[lane] = r;
+      if (a.rms && blockIdx.y == 0 && lane < nh) a.rms[t0 + lane] = r;
     }
-    if (st + 1u < nstage) {
-      fill_store(st + 1u, buf ^ 1u);
-      __syncthreads();
+  }
+  // normalised rows xn = x * (1/r) * gamma (x without RmsNorm) in the x dtype (or bf16), zero padded to Dp,
+  // chunk f of the token block by expert group f mod gridDim.y: U chunks at a time, the first U
+  // requested before r is known
+  constexpr uint32_t U = 3;
+  const uint32_t wstart = tid + blockDim.x * blockIdx.y, wstep = blockDim.x * gridDim.y;
+  const uint32_t cpr = a.Dp / 8u, nch = a.xn ? nh * cpr : 0u;  // Dp is a multiple of 32
+  Chunk8<XT> nx[U];
+  float4 ng[U][2];
+  auto fetch = [&](uint32_t f0) {
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t f = min(f0 + u * wstep, nch - 1u), t = f / cpr, c0 = (f - t * cpr) * 8u, c = c0 < D ? c0 : 0u;
+      chunk_load(nx[u], (const XT *)a.x + (size_t)(t0 + t) * D + c);
+      ng[u][0] = *(const float4 *)(a.gamma + c);
+      ng[u][1] = *(const float4 *)(a.gamma + c + 4);
+    }
+  };
+  if (nch) fetch(wstart);
+  __syncthreads();  // rr visible
+  if (tid < kRouterTok * 16u) {
+    const uint32_t t = tid >> 4, e = tid & 15u;
+    const float *rd = red + ((t >> 2) * 16u + e) * 4u + (t & 3u);
+    float s4[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+      float v[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; ++u) v[u] = rd[(u * 4u + k) * 256u];
+      s4[k] = ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
+    }
+    const float v = (s4[0] + s4[2]) + (s4[1] + s4[3]);
+    if (t < nh && e0 + e < E) a.logits[(size_t)(t0 + t) * E + e0 + e] = (a.apply_norm ? v / rr[t] : v) + a.rb[e0 + e];
+  }
+  for (uint32_t f0 = wstart; f0 < nch; f0 += U * wstep) {
+    if (f0 != wstart) fetch(f0);
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t f = f0 + u * wstep;
+      if (f >= nch) continue;
+      const uint32_t t = f / cpr, c0 = (f - t * cpr) * 8u;
+      float v[8];
+      chunk_vals(nx[u], v);
+      const float g[8] = {ng[u][0].x, ng[u][0].y, ng[u][0].z, ng[u][0].w, ng[u][1].x, ng[u][1].y, ng[u][1].z, ng[u][1].w};
+      const float ir = a.apply_norm ? 1.0f / rr[t] : 1.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = c0 >= D ? 0.0f : a.apply_norm ? (v[j] * ir) * g[j] : v[j];
+      if (a.xn_bf16)
+        store8((uint16_t *)a.xn + (size_t)(t0 + t) * a.Dp + c0, v);
+      else
+        store8((XT *)a.xn + (size_t)(t0 + t) * a.Dp + c0, v);
+    }
+  }
+  // their two-term form (grouped GEMM) zero padded to the K-group length, shared out block by block
+  auto norm8 = [&](uint32_t t, uint32_t c0, float *v) {  // c0 < D: 8 whole values
+    Chunk8<XT> c;
+    chunk_load(c, (const XT *)a.x + (size_t)(t0 + t) * D + c0);
+    float u[8];
+    chunk_vals(c, u);
+    if (a.apply_norm) {
+      const float ir = 1.0f / rr[t];
+      const float4 g0 = *(const float4 *)(a.gamma + c0), g1 = *(const float4 *)(a.gamma + c0 + 4);
+      const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) u[j] = (u[j] * ir) * g[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = u[j];
+  };
+  if (a.xq.hi) {
+    const uint32_t nbk = a.xq.kq >> 5;
+    for (uint32_t f = wstart; f < nh * nbk; f += wstep) {
+      const uint32_t t = f / nbk, bk = f - t * nbk;
+      float v[32], amax = 0.0f;
+#pragma unroll
+      for (uint32_t q = 0; q < 4u; ++q) {
+        const uint32_t c0 = bk * 32u + 8u * q;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[8u * q + j] = 0.0f;
+        if (c0 < D) norm8(t, c0, v + 8u * q);
+      }
+#pragma unroll
+      for (int k = 0; k < 32; ++k) amax = fmaxf(amax, fabsf(v[k]));
+      const size_t row = t0 + t;
+      mx84_quantize32(v, amax, a.xq.hi + row * a.xq.kq + bk * 32u, a.xq.lo + row * (a.xq.kq / 2u) + bk * 16u,
+                      a.xq.shi + row * a.xq.ss + bk, a.xq.slo + row * a.xq.ss + bk);
     }
   }
 }
@@ -2222,21 +2193,13 @@ hipError_t configure_kernels() {
   BX_ATTR((down_combine1_kernel<1, float>));
   BX_ATTR((down_combine1_kernel<2, float>));
   BX_ATTR((router_kernel<float, float, true>));
-  BX_ATTR((router_kernel<float, uint16_t, true>));
-  BX_ATTR((router_kernel<uint16_t, float, true>));
-  BX_ATTR((router_kernel<uint16_t, uint16_t, true>));
   BX_ATTR((router_kernel<float, float, false>));
+  BX_ATTR((router_kernel<float, uint16_t, true>));
   BX_ATTR((router_kernel<float, uint16_t, false>));
+  BX_ATTR((router_kernel<uint16_t, float, true>));
   BX_ATTR((router_kernel<uint16_t, float, false>));
+  BX_ATTR((router_kernel<uint16_t, uint16_t, true>));
   BX_ATTR((router_kernel<uint16_t, uint16_t, false>));
-  BX_ATTR((router_rows_kernel<float, float, 2>));
-  BX_ATTR((router_rows_kernel<float, float, 4>));
-  BX_ATTR((router_rows_kernel<float, uint16_t, 2>));
-  BX_ATTR((router_rows_kernel<float, uint16_t, 4>));
-  BX_ATTR((router_rows_kernel<uint16_t, float, 2>));
-  BX_ATTR((router_rows_kernel<uint16_t, float, 4>));
-  BX_ATTR((router_rows_kernel<uint16_t, uint16_t, 2>));
-  BX_ATTR((router_rows_kernel<uint16_t, uint16_t, 4>));
   BX_ATTR(dispatch_kernel);
   BX_ATTR((expert_gemv_kernel<1, true, uint16_t, kGateUpSplit, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, 1, false>));
@@ -2250,38 +2213,25 @@ hipError_t configure_kernels() {
   return err;
 }
 
+hipError_t launch_router_mfma(const RouterArgs &a, bool x_bf16, bool w_bf16, hipStream_t s) {
+  if (a.n == 0 || a.D == 0 || a.D % 8u != 0 || a.E == 0 ||
+      ((((uintptr_t)a.x | (uintptr_t)a.rw | (uintptr_t)a.gamma) & 15u) != 0) || (a.xn && a.Dp % 8u != 0) ||
+      (a.xq.hi && a.xq.kq % 32u != 0))
+    return hipErrorInvalidValue;
+  const dim3 grid((a.n + kRouterTok - 1u) / kRouterTok, (a.E + 15u) / 16u), block(64 * kRouterWaves);
+  if (x_bf16)
+    return w_bf16 ? launch_kernel(router_mfma_kernel<uint16_t, uint16_t>, grid, block, 0, s, a)
+                  : launch_kernel(router_mfma_kernel<uint16_t, float>, grid, block, 0, s, a);
+  return w_bf16 ? launch_kernel(router_mfma_kernel<float, uint16_t>, grid, block, 0, s, a)
+                : launch_kernel(router_mfma_kernel<float, float>, grid, block, 0, s, a);
+}
+
 template <typename XT, typename WT>
 static void router_launch(const RouterArgs &a, bool vec, dim3 grid, size_t lds, hipStream_t s) {
   if (vec)
     (void)launch_kernel(router_kernel<XT, WT, true>, grid, dim3(kRouterThreads), lds, s, a);
   else
     (void)launch_kernel(router_kernel<XT, WT, false>, grid, dim3(kRouterThreads), lds, s, a);
-}
-
-template <typename XT, typename WT>
-static void rows_launch(const RouterArgs &a, int tokens_per_wave, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
-  if (tokens_per_wave == 4)
-    (void)launch_kernel(router_rows_kernel<XT, WT, 4>, grid, block, lds, s, a);
-  else
-    (void)launch_kernel(router_rows_kernel<XT, WT, 2>, grid, block, lds, s, a);
-}
-
-hipError_t launch_router_rows(const RouterArgs &a, bool x_bf16, bool w_bf16, int tokens_per_wave, hipStream_t s) {
-  if (tokens_per_wave != 2 && tokens_per_wave != 4) return hipErrorInvalidValue;
-  if (a.D % 8u != 0 || a.D > kRowsSpan || (a.xn && a.Dp > kRowsSpan) || (a.xq.hi && a.xq.kq > kRowsSpan))
-    return hipErrorInvalidValue;
-  const uint32_t tpb = (uint32_t)tokens_per_wave * (kRowsThreads / 64u);
-  const dim3 grid((a.n + tpb - 1) / tpb), block(kRowsThreads);
-  const size_t lds = router_rows_lds_bytes();
-  if (x_bf16 && w_bf16)
-    rows_launch<uint16_t, uint16_t>(a, tokens_per_wave, grid, block, lds, s);
-  else if (x_bf16)
-    rows_launch<uint16_t, float>(a, tokens_per_wave, grid, block, lds, s);
-  else if (w_bf16)
-    rows_launch<float, uint16_t>(a, tokens_per_wave, grid, block, lds, s);
-  else
-    rows_launch<float, float>(a, tokens_per_wave, grid, block, lds, s);
-  return hipGetLastError();
 }
 
 hipError_t launch_router(const RouterArgs &a, bool x_bf16, bool w_bf16, bool vec, hipStream_t s) {

@@ -54,7 +54,7 @@ struct RouterArgs {
   uint32_t n, D, Dpad, Dp, E, tb, epw;
   float eps;
   int apply_norm;
-  int xn_bf16;        // xn rows rounded to bf16 (nearest even) whatever the x dtype (router_kernel)
+  int xn_bf16;        // xn rows rounded to bf16 (nearest even) whatever the x dtype
 };
 
 // Top-k + softmax per token (one wave per token) from logits [n, E].
@@ -332,11 +332,6 @@ __host__ __device__ inline size_t gemv_launch_lds_bytes(int nt, uint32_t mt_max,
 constexpr uint32_t kGemvKgPerWave = 6;  // K-groups per wave per step (6 KiB of weights in flight)
 
 constexpr uint32_t kRouterThreads = 256;
-// router_rows_kernel from this batch size on: its time is one workgroup's pass over all E router
-// rows (37 us at E = 32, 104 us at E = 128, D = 2880) while router_kernel's grows with n * E;
-// measured crossover between 1000 and 1200 tokens for both E
-constexpr uint32_t kRouterRowsMinTokens = 1152;
-constexpr uint32_t kRowsThreads = 512;
 constexpr uint32_t kTopkThreads = 512;
 constexpr uint32_t kDispatchThreads = 1024;
 constexpr uint32_t kDispatchChunk = 256;           // dispatch_wide_kernel: tokens per workgroup
@@ -355,9 +350,8 @@ constexpr uint32_t kMaxExperts = 256;
 constexpr uint32_t kSmallRouteMaxTokens = 16;  // decode-sized batches: one-workgroup routing kernel
 
 hipError_t launch_router(const RouterArgs &a, bool x_bf16, bool w_bf16, bool vec, hipStream_t s);
-// router_rows_kernel: D % 8 == 0 and D, Dp (with xn) and xq.kq (with xq) <= 512 * kFrontChunks,
-// 16-byte aligned x and router rows; 2 or 4 tokens per wave (16 or 32 per workgroup)
-hipError_t launch_router_rows(const RouterArgs &a, bool x_bf16, bool w_bf16, int tokens_per_wave, hipStream_t s);
+// router_mfma_kernel: D % 8 == 0, 16-byte aligned x, router rows and gamma
+hipError_t launch_router_mfma(const RouterArgs &a, bool x_bf16, bool w_bf16, hipStream_t s);
 hipError_t launch_small_route(const SmallRouteArgs &a, hipStream_t s);
 hipError_t launch_router_small(const FrontArgs &a, bool x_bf16, bool w_bf16, hipStream_t s);
 hipError_t launch_router_front(const PreFrontArgs &a, bool w_bf16, hipStream_t s);

@@ -555,8 +555,11 @@ burnext_status check_launch(hipError_t e, const char *what) {
   return BURNEXT_OK;
 }
 
-// Router logits (and r per token when normalising) into the workspace: router_rows_kernel for
-// batches of kRouterRowsMinTokens tokens or more whose rows fit its registers, router_kernel else.
+// Router logits (and r per token when normalising) into the workspace: router_mfma_kernel from
+// kRouterMfmaMinLogits logits on for rows it can read in 16-byte pieces, router_kernel else (its chain of
+// round trips is shorter while the grid does not fill the CUs: E = 32 8 / 15 us at 45 tokens, 15 / 18 at 523,
+// 33 / 19 at 1024; E = 128 11 / 14 at 64 tokens, 19 / 15 at 200, 48 / 17 at 512).
+constexpr uint64_t kRouterMfmaMinLogits = 20480;
 burnext_status run_router(burnext_moe_layer *L, const void *x, bool x_bf16, uint64_t n, bool norm, float *rms,
                           float *logits, void *xn, hipStream_t s, const QRows *xq = nullptr, bool xn_bf16 = false) {
   RouterArgs ra{};
@@ -580,14 +583,9 @@ burnext_status run_router(burnext_moe_layer *L, const void *x, bool x_bf16, uint
   ra.eps = L->eps;
   ra.apply_norm = norm ? 1 : 0;
   const bool vec = L->D % 8 == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)ra.rw & 15u) == 0;
-  const uint32_t lim = 512u * kFrontChunks;
-  const bool rows = vec && n >= kRouterRowsMinTokens && L->D <= lim && (!xn || L->Dp <= lim) &&
-                    (!xq || !xq->hi || xq->kq <= lim) && !xn_bf16;  // (bf16 rows: router_kernel)
   ProfScope ps(L, s, kKRouter);
-  // 4 tokens per wave (32 per workgroup) once that still gives every CU a workgroup: half the LDS
-  // reads per token (measured: 120B T = 8192 206 -> 171 us; slower while the grid is short of the CUs)
-  const int tpw = n >= 32ull * (uint64_t)L->num_cus ? 4 : 2;
-  return check_launch(rows ? launch_router_rows(ra, x_bf16, w_bf16, tpw, s) : launch_router(ra, x_bf16, w_bf16, vec, s),
+  const bool mfma = vec && n * L->E >= kRouterMfmaMinLogits;
+  return check_launch(mfma ? launch_router_mfma(ra, x_bf16, w_bf16, s) : launch_router(ra, x_bf16, w_bf16, vec, s),
                       "router kernel launch");
 }
 
