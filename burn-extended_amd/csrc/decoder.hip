@@ -1267,12 +1267,14 @@ struct GWs {
 
 // The streaming LM head (lm_stream_kernel) serves batches of at most kLmMaxB rows whose d_model
 // fits its LDS staging (K <= kLmMaxK, K % 8 == 0, a batch of at least 1 KiB for the dummy refills)
-// and vocabularies of at least one row tile per wave of one workgroup (and fewer than 2^32
-// K-groups: lm_fix_kernel's 32-bit cuts).
+// and vocabularies that give at least half the CUs a workgroup (a wave takes at least one row tile:
+// 16 384 rows are 64 workgroups), with fewer than 2^32 K-groups (lm_fix_kernel's 32-bit cuts).
+// Decode steps with it against the K-split GEMV, d_model 2880, 1 / 8 rows: 96 / 108 against 85 / 95 us at
+// 16 384, 102 / 112 and 99 / 112 at 32 768, 112 / 125 and 114 / 134 at 50 001, 157 / 173 and 158 / 186 at 100 000.
 bool lm_stream_ok(const burnext_gptoss &M, uint32_t B) {
   const uint32_t K = M.lm.K;
   return B >= 1u && B <= kLmMaxB && K <= kLmMaxK && K % 8u == 0u && (uint64_t)B * K * 4u >= 1024u &&
-         M.lm.ntiles >= kLmWaves && (uint64_t)M.lm.ntiles * M.lm.nkg < (1ull << 32);
+         2ull * M.lm.ntiles >= (uint64_t)kLmWaves * (uint32_t)M.num_cus && (uint64_t)M.lm.ntiles * M.lm.nkg < (1ull << 32);
 }
 // Its waves: one workgroup per CU, at most one wave per row tile (so every run spans at least nkg
 // K-groups and a tile is cut at most once).
