@@ -36,9 +36,9 @@ namespace {
 //     of bank conflicts (slot c ^ ((t >> 2) & 3) measured 2-way conflicted on gfx950).
 // The B scales come in blocks of 4 K-groups, outside the stage ring: two slots (double buffer)
 // of [term 2][token 64][16 bytes] (byte 4 k + g = scale of K [32 g, 32 g + 32) of K-group 4 j + k
-// of block j).  One 16-byte fill instruction per wave and block (32 tokens of one term, the
-// upper 32 lanes masked) replaces four gathers of 4-byte pieces: the gathers' per-row cost in the
-// address and data paths took 35 of gate_up's 412 us at C3.
+// of block j).  One 16-byte fill instruction per wave and block (64 tokens of one
+// term) replaces four gathers of 4-byte pieces: the gathers' per-row cost in the address and data
+// paths took 35 of gate_up's 412 us at C3.
 constexpr uint32_t kRowTiles = kGemmRows / 16u;
 constexpr uint32_t kBHi = 8u * kGemmTok * 16u;
 constexpr uint32_t kBData = kBHi + 4u * kGemmTok * 16u;
@@ -89,77 +89,25 @@ __device__ __forceinline__ void ring_barrier() {
 
 size_t gemm_lds_bytes() { return (size_t)kStages * kStage + kScaleRing + 2 * kGemmTok * 4 + 64 + 2 * (kMaxExperts + 1) * 4; }
 
-// Work item of workgroup b: blockIdx is remapped so that the workgroups of one XCD (b mod 8)
-// take a contiguous run of Q = ceil(N / 8) of the N realised items (N = nrb * token tiles, read
-// from tile_off[E]; the grid is sized for the most tiles routing can produce, and sizing the runs
-// by the grid left the last XCD a small remainder while the other seven did all the work).  Items
-// go in groups of 8 token tiles: row block rb of the group's tiles, tiles fastest, so the ~64
-// workgroups an XCD runs at once share about 8 row blocks of weights and 8 tiles of activations
-// in its L2 (gate_up HBM reads 2.1 -> 1.0 GB per launch at C3 against row blocks fastest).
-// A workgroup (4 waves; two workgroups per CU, whose K-loops drift apart, so one's LDS reads
-// and waits overlap the other's MFMAs) computes kGemmRows weight rows (16 row tiles) x kGemmTok
-// tokens; wave w computes rows 64 w .. 64 w + 63 (4 x 4 MFMA tiles of 16 x 16, two terms each).
-// Weights go straight from the tiled layout into registers, two K-groups ahead (two register
-// sets), their scales from the GEMM scale copy (one 16-byte load per wave and 4 K-groups, the byte
-// picked by the MFMA's op_sel; the K-loop is unrolled by 4 for it); activations stream through a 5-stage LDS ring filled by direct-to-LDS loads four
-// K-groups ahead (3 instructions per wave per stage, and one per 4 K-groups for the scales);
-// one barrier per K-group.
-template <bool GATE_UP>
-__global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  uint8_t *scl = smem + kStages * kStage;                      // B scale blocks [slot 2]
-  int32_t *rows_l = (int32_t *)(scl + kScaleRing);              // [kGemmTok] B row, -1 = none
-  int32_t *slot_l = rows_l + kGemmTok;                     // [kGemmTok] down: slot
-  int32_t *info_l = slot_l + kGemmTok;                     // [0] expert [1] tile of it
-  int32_t *toff_l = info_l + 16;                           // [E + 1] tile_off
-  int32_t *soff_l = toff_l + kMaxExperts + 1;              // [E + 1] seg_off
+namespace {
+// What a workgroup's item is (read by the prologue) and its LDS.
+struct GemmItem {
+  int e, seg0;
+  uint32_t rb, m0, ntok;
+  int32_t slot_own;  // down: this thread's output slot, its load still in flight
+  uint8_t *smem;
+  int32_t *rows_l, *slot_l;
+};
 
-  // one round trip for both prefixes (E + 1 <= 257 entries each), then the item and its expert
-  // from LDS
-  for (uint32_t t = threadIdx.x; t <= a.E; t += blockDim.x) {
-    toff_l[t] = a.tile_off[t];
-    soff_l[t] = a.seg_off[t];
-  }
-  if (threadIdx.x == 0) info_l[0] = -1;
-  __syncthreads();
-  const uint32_t b = blockIdx.x;
-  const uint32_t NT = (uint32_t)toff_l[a.E];
-  const uint32_t N = a.nrb * NT, Q = (N + 7u) / 8u;  // 8 * Q <= gridDim.x
-  const uint32_t it = (b & 7u) * Q + (b >> 3);
-  if ((b >> 3) >= Q || it >= N) return;  // workgroup-uniform: no item
-  // items in groups of 8 token tiles: row block rb of the group's tiles, tiles fastest
-  const uint32_t grp = it / (8u * a.nrb), r = it - grp * 8u * a.nrb;
-  const uint32_t gsz = min(8u, NT - grp * 8u);
-  const uint32_t rb = r / gsz, gt = grp * 8u + (r - rb * gsz);
-  for (uint32_t e = threadIdx.x; e < a.E; e += blockDim.x) {
-    const uint32_t lo = (uint32_t)toff_l[e], hi = (uint32_t)toff_l[e + 1];
-    if (gt >= lo && gt < hi) {
-      info_l[0] = (int32_t)e;
-      info_l[1] = (int32_t)(gt - lo);
-    }
-  }
-  __syncthreads();
-  const int e = info_l[0];
-  if (e < 0) return;  // workgroup-uniform: beyond the realised token tiles
-  const int seg0 = soff_l[e];
-  const uint32_t M = (uint32_t)(soff_l[e + 1] - seg0);
-  const uint32_t m0 = (uint32_t)info_l[1] * kGemmTok;
-  const uint32_t ntok = min(kGemmTok, M - m0);
-  // B rows: gate_up reads token rows (slot / topk of the segment entries, one more round trip);
-  // down reads the segment's own rows, and its output slots are needed only by the epilogue, so
-  // their load is waited for after the K-loop
-  static_assert(kGemmTok <= 256, "one segment entry per thread");
-  // every thread loads (clamped index: no branch around the load); entries >= ntok are dropped
-  const int32_t slot_own = a.perm[seg0 + (int32_t)min(m0 + threadIdx.x, M - 1u)];
-  if (threadIdx.x < kGemmTok) {
-    const uint32_t i = threadIdx.x;
-    if (GATE_UP)
-      rows_l[i] = i < ntok ? slot_own / (int32_t)a.topk : -1;
-    else
-      rows_l[i] = i < ntok ? seg0 + (int32_t)(m0 + i) : -1;
-  }
-  ring_barrier();  // rows_l written (LDS); down's slot load stays in flight
-
+// The item's K-loop and epilogue.  TT: token columns of 16 computed (2 or 3 for items of at most 32
+// or 48 tokens: fewer operand reads and MFMAs, and at 2 half the hi stage).  STREAM: nontemporal weights.
+template <bool GATE_UP, bool STREAM, int TT>
+__device__ __forceinline__ void gemm_body(const GemmArgs &a, const GemmItem &it) {
+  constexpr int kHi = (TT + 1) / 2;  // hi fill instructions of a stage (32 tokens each)
+  uint8_t *smem = it.smem, *scl = smem + kStages * kStage;
+  int32_t *rows_l = it.rows_l, *slot_l = it.slot_l;
+  const int e = it.e, seg0 = it.seg0, slot_own = it.slot_own;
+  const uint32_t rb = it.rb, m0 = it.m0, ntok = it.ntok;
   const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
   const uint32_t wr = wv;  // this wave's 64-row quarter of the workgroup's rows
   const uint32_t i16 = lane & 15u, q = lane >> 4;
@@ -186,8 +134,9 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   const int32_t rkl = rows_l[tkl];
   const size_t browl = (size_t)(rkl >= 0 ? rkl : rows_l[0]) * (kq / 2u);
   const uint32_t lchunk = ((lane & 3u) ^ ((tkl >> 2) & 2u)) * 16u;
-  // B scale blocks: term wv / 2, token 32 (wv % 2) + lane (lanes < 32)
-  const int32_t rsl = rows_l[32u * (wv & 1u) + (lane & 31u)];
+  // B scale blocks: term wv % 2, token lane (two waves write the same bytes: a load that half the lanes
+  // or waves skip is a branch, and the compiler then drains every load in flight before the next use)
+  const int32_t rsl = rows_l[lane];
   const size_t rows = (size_t)(rsl >= 0 ? rsl : rows_l[0]);
   // this wave's 4 row tiles (clamped to the expert's last) and their group in the GEMM's scale
   // copy (clamped to the last group: rows beyond the expert are never stored)
@@ -202,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   auto stage = [&](uint32_t kg, uint32_t p) {
     uint8_t *st = smem + p * kStage;
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {  // B hi codes: token group wv + 4 m
+    for (int m = 0; m < kHi; ++m) {  // B hi codes: token group wv + 4 m
       const uint32_t tg = wv + 4u * (uint32_t)m;
       const uint8_t *src = a.b.hi + (m ? browk1 : browk0) + kg * 128u + bchunk;
       __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + tg * 64u * 16u), 16, 0, 0);
@@ -214,16 +163,15 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   };
   // B scale block j (K-groups 4 j .. 4 j + 3) into slot p: 16 bytes per token and term
   auto stage_scales = [&](uint32_t j, uint32_t p) {
-    const uint8_t *src = (wv >= 2u ? a.b.slo : a.b.shi) + rows * ss + j * 16u;
-    if (lane < 32u)
-      __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(scl + p * kScaleSlot + wv * 512u), 16, 0, 0);
+    const uint8_t *src = ((wv & 1u) ? a.b.slo : a.b.shi) + rows * ss + j * 16u;
+    __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(scl + p * kScaleSlot + (wv & 1u) * 1024u), 16, 0, 0);
   };
 
-  f32x4_t acc[4][4];
+  f32x4_t acc[4][TT];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) acc[rt][tt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int tt = 0; tt < TT; ++tt) acc[rt][tt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
   // MFMA operands: the A operands (row tiles) of a K-group, and the B operands of one token tile.
   // The A scales of 4 K-groups come in one 16-byte load (dword rt: byte k = K-group 4 j + k of row
@@ -242,7 +190,8 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   auto load_a = [&](uint32_t kg, AFrag &f) {
     const uint32_t off = lane_ok(kg) ? kg * 1024u : 0u;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) f.A[rt] = *(const i32x4_t *)(arow[rt] + off);
+    for (int rt = 0; rt < 4; ++rt)
+      f.A[rt] = STREAM ? __builtin_nontemporal_load((const i32x4_t *)(arow[rt] + off)) : *(const i32x4_t *)(arow[rt] + off);
     __builtin_amdgcn_sched_barrier(0);  // the wait counts below assume this issue order
   };
   // A scales of K-groups 4 j .. 4 j + 3 (lanes beyond the blocks read scale byte 0)
@@ -297,17 +246,18 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   for (uint32_t j = 0; j < kStages - 1u; ++j) stage(min(j, nkg - 1u), j);
   stage_scales(0, 0);
   __builtin_amdgcn_sched_barrier(0);
-  AFrag ar0, ar1;
+  AFrag ar[2];
   i32x4_t sa_cur, sa_nxt;  // A scales of the current block, and of the next (loaded at position 2)
-  load_a(0, ar0);
+  load_a(0, ar[0]);
   load_as(0, sa_cur);
-  load_a(min(1u, nkg - 1u), ar1);
+  load_a(min(1u, nkg - 1u), ar[1]);
   __builtin_amdgcn_s_waitcnt(vmcnt_only(4));  // A(0), its scales and every B stage before them landed
   ring_barrier();
   // K-group kg at position P = kg mod 4 of its scale block (a compile-time constant: the block
   // loads, one per 4 K-groups, change the wait count)
-  auto iter = [&](uint32_t kg, AFrag &ar, auto P) {
+  auto iter = [&](uint32_t kg, auto P) {
     constexpr uint32_t kP = decltype(P)::value;
+    AFrag &A = ar[kP & 1u];
     stage(min(kg + kStages - 1u, nkg - 1u), (kg + kStages - 1u) % kStages);  // the slot every wave left
     // the next scale block into the slot of the previous one (every wave is past its last K-group)
     if constexpr (kP == 0u) stage_scales(min((kg >> 2) + 1u, (nkg - 1u) >> 2), ((kg >> 2) + 1u) & 1u);
@@ -320,17 +270,17 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
     __builtin_amdgcn_s_setprio(1);
     read_b(st, sc, 0, b0);
     read_b(st, sc, 1, b1);
-    mma(ar, sa_cur, b0, 0, P);
-    read_b(st, sc, 2, b0);
-    mma(ar, sa_cur, b1, 1, P);
-    read_b(st, sc, 3, b1);
-    mma(ar, sa_cur, b0, 2, P);
-    mma(ar, sa_cur, b1, 3, P);
+    mma(A, sa_cur, b0, 0, P);
+    if constexpr (TT > 2) read_b(st, sc, 2, b0);
+    mma(A, sa_cur, b1, 1, P);
+    if constexpr (TT > 3) read_b(st, sc, 3, b1);
+    if constexpr (TT > 2) mma(A, sa_cur, b0, 2, P);
+    if constexpr (TT > 3) mma(A, sa_cur, b1, 3, P);
     // schedule: tile 0's operand reads, then each next tile's reads one by one between the MFMAs
     // of the tile before it (gate_up 474 -> 468 us at C3 against the compiler's own order)
     __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);  // 0x100: LDS reads, 0x008: MFMAs
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
+    for (int t = 0; t < TT - 1; ++t) {
 #pragma unroll
       for (int i = 0; i < 5; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -340,13 +290,13 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
     __builtin_amdgcn_s_setprio(0);
-    load_a(min(kg + 2u, nkg - 1u), ar);
+    load_a(min(kg + 2u, nkg - 1u), A);
     // at position 2, the next block's A scales (needed from K-group kg + 2 on)
     if constexpr (kP == 2u) load_as(min((kg >> 2) + 1u, nkq - 1u), sa_nxt);
     // issued after A(kg + 1): B(kg + 4), at position 0 a B scale block, A(kg + 2) and at position 2
-    // the A scale block (3 [+ 1] + 4 [+ 1]); B(kg + 1) and kg + 1's B scale block went out before
-    // A(kg + 1).  At position 3 the A scale block issued after A(kg + 1) is waited for too (3 + 4).
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(kP == 0u || kP == 2u ? 8 : 7));
+    // the A scale block (kHi + 1 [+ 1] + 4 [+ 1]); B(kg + 1) and kg + 1's B scale block went out before
+    // A(kg + 1).  At position 3 the A scale block issued after A(kg + 1) is waited for too (kHi + 1 + 4).
+    __builtin_amdgcn_s_waitcnt(vmcnt_only((kP == 0u || kP == 2u ? 6 : 5) + kHi));
     if constexpr (kP == 3u) sa_cur = sa_nxt;
     ring_barrier();
   };
@@ -356,14 +306,14 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
   using P3 = std::integral_constant<uint32_t, 3>;
   uint32_t kg = 0;
   for (; kg + 3u < nkg; kg += 4u) {
-    iter(kg, ar0, P0{});
-    iter(kg + 1u, ar1, P1{});
-    iter(kg + 2u, ar0, P2{});
-    iter(kg + 3u, ar1, P3{});
+    iter(kg, P0{});
+    iter(kg + 1u, P1{});
+    iter(kg + 2u, P2{});
+    iter(kg + 3u, P3{});
   }
-  if (kg < nkg) iter(kg, ar0, P0{});
-  if (kg + 1u < nkg) iter(kg + 1u, ar1, P1{});
-  if (kg + 2u < nkg) iter(kg + 2u, ar0, P2{});
+  if (kg < nkg) iter(kg, P0{});
+  if (kg + 1u < nkg) iter(kg + 1u, P1{});
+  if (kg + 2u < nkg) iter(kg + 2u, P2{});
   __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // the trailing reloads have landed
   if (!GATE_UP) {
     if (threadIdx.x < kGemmTok) slot_l[threadIdx.x] = threadIdx.x < ntok ? slot_own : -1;
@@ -383,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
     uint8_t *hi_l = ep, *lo_l = ep + kGemmTok * kHs, *sc_l = ep + kGemmTok * (kHs + kLs);
     const uint32_t fb = rb * (kGemmRows / 2u) + wr * 32u;
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
+    for (int tt = 0; tt < TT; ++tt) {
       const uint32_t tok = (uint32_t)tt * 16u + i16;
       float o[8];
       float amax = 0.0f;
@@ -471,7 +421,7 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
     constexpr uint32_t kOs = 264u;  // padded row stride (elements)
     uint16_t *o_l = (uint16_t *)ep;
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
+    for (int tt = 0; tt < TT; ++tt) {
       const uint32_t tok = (uint32_t)tt * 16u + i16;
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
@@ -501,23 +451,115 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
     }
   }
 }
+}  // namespace
+
+// Work item of workgroup b: blockIdx is remapped so that the workgroups of one XCD (b mod 8)
+// take a contiguous run of Q = ceil(N / 8) of the N realised items (N = nrb * token tiles, read
+// from tile_off[E]; the grid is sized for the most tiles routing can produce, and sizing the runs
+// by the grid left the last XCD a small remainder while the other seven did all the work).  Items
+// go in groups of 8 token tiles: row block rb of the group's tiles, tiles fastest, so the ~64
+// workgroups an XCD runs at once share about 8 row blocks of weights and 8 tiles of activations
+// in its L2 (gate_up HBM reads 2.1 -> 1.0 GB per launch at C3 against row blocks fastest).
+// A workgroup (4 waves; two workgroups per CU, whose K-loops drift apart, so one's LDS reads
+// and waits overlap the other's MFMAs) computes kGemmRows weight rows (16 row tiles) x kGemmTok
+// tokens; wave w computes rows 64 w .. 64 w + 63 (4 x 4 MFMA tiles of 16 x 16, two terms each).
+// No load of the K-loop is behind a branch or an exec mask: with the scale blocks' fill masked to half
+// the lanes the compiler drained every load in flight once per 4 K-groups (C3 gate_up 403 -> 388 us,
+// down 219 -> 208; 120B 4096 tokens 511 -> 485, 271 -> 254).  Items of at most 32 or 48 tokens compute 2 or 3
+// token columns (120B 512 tokens gate_up 244 -> 224 us, streamed 211).
+// Weights go straight from the tiled layout into registers, two K-groups ahead (two register
+// sets), their scales from the GEMM scale copy (one 16-byte load per wave and 4 K-groups, the byte
+// picked by the MFMA's op_sel; the K-loop is unrolled by 4 for it); activations stream through a 5-stage LDS ring filled by direct-to-LDS loads four
+// K-groups ahead (3 instructions per wave per stage, and one per 4 K-groups for the scales);
+// one barrier per K-group.
+template <bool GATE_UP, bool STREAM>
+__global__ __launch_bounds__(256, 2) void expert_gemm_kernel(GemmArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  // stage ring, B scale blocks [slot 2], then
+  int32_t *rows_l = (int32_t *)(smem + kStages * kStage + kScaleRing);  // [kGemmTok] B row, -1 = none
+  int32_t *slot_l = rows_l + kGemmTok;                     // [kGemmTok] down: slot
+  int32_t *info_l = slot_l + kGemmTok;                     // [0] expert [1] tile of it
+  int32_t *toff_l = info_l + 16;                           // [E + 1] tile_off
+  int32_t *soff_l = toff_l + kMaxExperts + 1;              // [E + 1] seg_off
+
+  // one round trip for both prefixes (E + 1 <= 257 entries each), then the item and its expert
+  // from LDS
+  for (uint32_t t = threadIdx.x; t <= a.E; t += blockDim.x) {
+    toff_l[t] = a.tile_off[t];
+    soff_l[t] = a.seg_off[t];
+  }
+  if (threadIdx.x == 0) info_l[0] = -1;
+  __syncthreads();
+  const uint32_t b = blockIdx.x;
+  const uint32_t NT = (uint32_t)toff_l[a.E];
+  const uint32_t N = a.nrb * NT, Q = (N + 7u) / 8u;  // 8 * Q <= gridDim.x
+  const uint32_t it = (b & 7u) * Q + (b >> 3);
+  if ((b >> 3) >= Q || it >= N) return;  // workgroup-uniform: no item
+  // items in groups of 8 token tiles: row block rb of the group's tiles, tiles fastest
+  const uint32_t grp = it / (8u * a.nrb), r = it - grp * 8u * a.nrb;
+  const uint32_t gsz = min(8u, NT - grp * 8u);
+  const uint32_t rb = r / gsz, gt = grp * 8u + (r - rb * gsz);
+  for (uint32_t e = threadIdx.x; e < a.E; e += blockDim.x) {
+    const uint32_t lo = (uint32_t)toff_l[e], hi = (uint32_t)toff_l[e + 1];
+    if (gt >= lo && gt < hi) {
+      info_l[0] = (int32_t)e;
+      info_l[1] = (int32_t)(gt - lo);
+    }
+  }
+  __syncthreads();
+  const int e = info_l[0];
+  if (e < 0) return;  // workgroup-uniform: beyond the realised token tiles
+  const int seg0 = soff_l[e];
+  const uint32_t M = (uint32_t)(soff_l[e + 1] - seg0);
+  const uint32_t m0 = (uint32_t)info_l[1] * kGemmTok;
+  const uint32_t ntok = min(kGemmTok, M - m0);
+  // B rows: gate_up reads token rows (slot / topk of the segment entries, one more round trip);
+  // down reads the segment's own rows, and its output slots are needed only by the epilogue, so
+  // their load is waited for after the K-loop
+  static_assert(kGemmTok <= 256, "one segment entry per thread");
+  // every thread loads (clamped index: no branch around the load); entries >= ntok are dropped
+  const int32_t slot_own = a.perm[seg0 + (int32_t)min(m0 + threadIdx.x, M - 1u)];
+  if (threadIdx.x < kGemmTok) {
+    const uint32_t i = threadIdx.x;
+    if (GATE_UP)
+      rows_l[i] = i < ntok ? slot_own / (int32_t)a.topk : -1;
+    else
+      rows_l[i] = i < ntok ? seg0 + (int32_t)(m0 + i) : -1;
+  }
+  ring_barrier();  // rows_l written (LDS); down's slot load stays in flight
+
+  const GemmItem item{e, seg0, rb, m0, ntok, slot_own, smem, rows_l, slot_l};
+  if (ntok <= 32u)
+    gemm_body<GATE_UP, STREAM, 2>(a, item);
+  else if (ntok <= 48u)
+    gemm_body<GATE_UP, STREAM, 3>(a, item);
+  else
+    gemm_body<GATE_UP, STREAM, 4>(a, item);
+}
 
 hipError_t configure_gemm_kernels() {
   const int lds = (int)gemm_lds_bytes();
-  hipError_t e1 = hipFuncSetAttribute((const void *)expert_gemm_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipError_t e2 = hipFuncSetAttribute((const void *)expert_gemm_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  return e1 != hipSuccess ? e1 : e2;
+  hipError_t err = hipSuccess;
+  for (const void *f : {(const void *)expert_gemm_kernel<true, false>, (const void *)expert_gemm_kernel<true, true>,
+                        (const void *)expert_gemm_kernel<false, false>, (const void *)expert_gemm_kernel<false, true>}) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (err == hipSuccess) err = e;
+  }
+  return err;
 }
 
-hipError_t launch_gemm(const GemmArgs &a, bool gate_up, uint32_t grid, hipStream_t s) {
+hipError_t launch_gemm(const GemmArgs &a, bool gate_up, bool stream, uint32_t grid, hipStream_t s) {
   // B scale rows hold whole 16-byte blocks of 4 K-groups (ss >= kq / 32, a multiple of 16)
   if (grid == 0 || (grid & 7u) != 0 || a.nrb == 0 || a.b.kq % 128u != 0 || a.b.ss % 16u != 0 || a.b.ss * 32u < a.b.kq)
     return hipErrorInvalidValue;
   if (gate_up && (a.act.kq % 128u != 0 || a.act.ss * 32u < a.act.kq)) return hipErrorInvalidValue;
+  const dim3 g(grid), blk(64 * kWaves);
   if (gate_up)
-    (void)launch_kernel(expert_gemm_kernel<true>, dim3(grid), dim3(64 * kWaves), gemm_lds_bytes(), s, a);
+    (void)(stream ? launch_kernel(expert_gemm_kernel<true, true>, g, blk, gemm_lds_bytes(), s, a)
+                  : launch_kernel(expert_gemm_kernel<true, false>, g, blk, gemm_lds_bytes(), s, a));
   else
-    (void)launch_kernel(expert_gemm_kernel<false>, dim3(grid), dim3(64 * kWaves), gemm_lds_bytes(), s, a);
+    (void)(stream ? launch_kernel(expert_gemm_kernel<false, true>, g, blk, gemm_lds_bytes(), s, a)
+                  : launch_kernel(expert_gemm_kernel<false, false>, g, blk, gemm_lds_bytes(), s, a));
   return hipGetLastError();
 }
 

@@ -1412,7 +1412,7 @@ __device__ __forceinline__ bool gemv_share(uint32_t g, uint32_t G, uint32_t na, 
   return cnt > 0u;
 }
 
-// Single-token batches that touch few experts (more tokens or experts: tile_gemm.hip).
+// Single-token batches (more tokens: tile_gemm.hip).
 // Work split.  Grid of G workgroups (as many as stay resident); workgroup g owns the units
 // gemv_share gives it, wave w every 4th of them from its w-th.  A unit is a row tile or (down with
 // ksplit) one of ksplit fixed K-parts of a row tile (unit u: part u / nrt of row tile u mod nrt).
@@ -2201,6 +2201,8 @@ hipError_t configure_kernels() {
   BX_ATTR((router_kernel<uint16_t, uint16_t, true>));
   BX_ATTR((router_kernel<uint16_t, uint16_t, false>));
   BX_ATTR(dispatch_kernel);
+  BX_ATTR((expert_gemv_kernel<1, true, uint16_t, 1, false>));
+  BX_ATTR((expert_gemv_kernel<2, true, float, 1, true>));
   BX_ATTR((expert_gemv_kernel<1, true, uint16_t, kGateUpSplit, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, 1, false>));
   BX_ATTR((expert_gemv_kernel<1, false, float, kDownSplit, false>));
@@ -2323,7 +2325,9 @@ hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t s) {
 template <int NT, typename XT, bool PK>
 static hipError_t launch_gemv_t(const GemvArgs &a, bool gate_up, dim3 g, size_t lds, hipStream_t s) {
   const dim3 block(kGemvThreads);
-  if (gate_up) return launch_kernel(expert_gemv_kernel<NT, true, XT, kGateUpSplit, PK>, g, block, lds, s, a);
+  if (gate_up)
+    return a.ksplit > 1u ? launch_kernel(expert_gemv_kernel<NT, true, XT, kGateUpSplit, PK>, g, block, lds, s, a)
+                         : launch_kernel(expert_gemv_kernel<NT, true, XT, 1, PK>, g, block, lds, s, a);
   if (a.ksplit == kDownSplitFew) return launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplitFew, PK>, g, block, lds, s, a);
   if (a.ksplit == kDownSplit) return launch_kernel(expert_gemv_kernel<NT, false, float, kDownSplit, PK>, g, block, lds, s, a);
   return launch_kernel(expert_gemv_kernel<NT, false, float, 1, PK>, g, block, lds, s, a);
@@ -2338,7 +2342,7 @@ hipError_t launch_gemv(const GemvArgs &a, int nt, bool gate_up, bool x_bf16, uin
     return hipErrorInvalidValue;
   const size_t lds = gemv_launch_lds_bytes(nt, a.mt_max, a.nb, a.nrec, gate_up && a.ksplit > 1u);
   if (!gate_up && a.ksplit > 1u && a.ksplit != kDownSplit && a.ksplit != kDownSplitFew) return hipErrorInvalidValue;
-  if (gate_up && a.ksplit != kGateUpSplit) return hipErrorInvalidValue;
+  if (gate_up && a.ksplit > 1u && a.ksplit != kGateUpSplit) return hipErrorInvalidValue;
   if (nt == 1 && (x_bf16 || !gate_up)) return launch_gemv_t<1, uint16_t, false>(a, gate_up, g, lds, s);
   if (nt == 2 && (!x_bf16 || !gate_up) && 2u * a.mt_max <= 16u)  // both terms in one MFMA's columns
     return launch_gemv_t<2, float, true>(a, gate_up, g, lds, s);

@@ -376,7 +376,7 @@ hipError_t launch_fused(const FusedArgs &a, const FusedGeom &g, int nt, bool x_b
 // parts part_stride apart, their count as the fused kernel set it (CombineArgs.num_active)
 hipError_t launch_combine_slices(const CombineArgs &a, bool x_bf16, hipStream_t s);
 hipError_t configure_fused_kernels();
-hipError_t launch_gemm(const GemmArgs &a, bool gate_up, uint32_t grid, hipStream_t s);
+hipError_t launch_gemm(const GemmArgs &a, bool gate_up, bool stream, uint32_t grid, hipStream_t s);
 hipError_t configure_gemm_kernels();
 size_t gemm_lds_bytes();
 hipError_t launch_tile(const TileArgs &a, const TileShape &t, int nt, bool gate_up, bool x_bf16, uint32_t grid, hipStream_t s);

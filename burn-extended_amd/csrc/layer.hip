@@ -294,11 +294,11 @@ struct GemvCfg {
   uint32_t grid, nrec;
 };
 
-GemvCfg gemv_cfg(const burnext_moe_layer &L, int nt, bool gate_up) {
+GemvCfg gemv_cfg(const burnext_moe_layer &L, int nt, bool gate_up, bool split) {
   const TiledMx &t = gate_up ? L.w1 : L.w2;
   GemvCfg c{};
   c.nrec = std::min(L.E, L.K);
-  const size_t lds = gemv_launch_lds_bytes(nt, 1, t.nb, c.nrec, gate_up);
+  const size_t lds = gemv_launch_lds_bytes(nt, 1, t.nb, c.nrec, gate_up && split);
   const uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(4, (160 * 1024) / std::max<size_t>(lds, 1)));
   c.grid = (uint32_t)std::max<uint64_t>(c.nrec, std::min<uint64_t>((uint64_t)L.num_cus * per_cu, (uint64_t)c.nrec * t.nrt));
   return c;
@@ -331,20 +331,25 @@ inline bool gemm_regions(const burnext_moe_layer &L, uint64_t n) {
   return n >= kGemmMinTokens && n * L.K >= kGemmMinPerExpert * L.E;
 }
 
-// The expert projections by batch size: a single token that touches few experts (gate_up_split) by
-// the expert GEMVs; all others as tiles on bf16 MFMA (tile_gemm.hip: the GEMV's operands and
-// precision), except bf16 batches of
+// The expert projections by batch size: a single token by the expert GEMVs, which route it in their
+// prologue (a launch fewer than tiles: 18.5 / 20.5 us on a small layer); all others as tiles on bf16 MFMA
+// (tile_gemm.hip: the GEMV's operands and precision), except bf16 batches of
 // kMxMinTokens tokens and kMxMinPerExpert routed tokens per expert, which run the grouped GEMM on the
 // block-scaled MFMA (its two activation terms carry about 2^-6 relative precision: bf16 rows only).
-// Tiles against the grouped GEMM per step, D = F = 2880, k = 4, bf16: E = 32 109 / 134 us at 64 tokens,
-// 125 / 135 at 128, 129 / 136 at 160, 141 / 139 at 200, 162 / 141 at 256; E = 128 322 / 384 at 128, 358 / 398
-// at 200, 400 / 415 at 300, 428 / 428 at 400, 448 / 439 at 512.  Against GEMV passes of 8 .. 14 token rows:
-// E = 32 bf16 98 / 107 us at 17 tokens, 101 / 113 at 45, 108 / 130 at 63, f32 115 / 133 at 17 and 340 / 1085 at
-// 523; E = 128 bf16 278 / 308 at 64, 310 / 376 at 100.  Decode sizes, tiles of 16 tokens x 128 rows against
-// GEMV passes of 8 (bf16) and 4 (f32) rows in K-halves: E = 32 bf16 39 / 50 us at 2 tokens, 53 / 62 at 4,
-// 67 / 74 at 8, 87 / 95 at 16, f32 46 / 52 at 2, 71 / 73 at 8, 92 / 113 at 16; 64-row tiles 38 / 54 / 71 / 92 (bf16).
-constexpr uint64_t kMxMinTokens = 192;
-constexpr uint64_t kMxMinPerExpert = 12;
+// Tiles against the grouped GEMM per step, D = F = 2880, k = 4, bf16: E = 32 109 / 110 us at 64 tokens,
+// 119 / 112 at 96, 126 / 115 at 128, 139 / 121 at 190; E = 128 322 / 317 at 128, 351 / 324 at 200, 390 / 343 at
+// 380.  Against GEMV passes of 8 .. 14 token rows: E = 32 bf16 98 / 107 us at 17 tokens, 101 / 113 at 45, 108 /
+// 130 at 63, f32 115 / 133 at 17 and 340 / 1085 at 523; E = 128 bf16 278 / 308 at 64, 310 / 376 at 100.  Decode
+// sizes, tiles of 16 tokens x 128 rows against GEMV passes of 8 (bf16) and 4 (f32) rows in K-halves: E = 32
+// bf16 39 / 50 us at 2 tokens, 53 / 62 at 4, 67 / 74 at 8, 87 / 95 at 16, f32 46 / 52 at 2, 71 / 73 at 8, 92 / 113
+// at 16; 64-row tiles 38 / 54 / 71 / 92 (bf16).
+constexpr uint64_t kMxMinTokens = 80;
+constexpr uint64_t kMxMinPerExpert = 4;
+// The grouped GEMM streams its weights past the caches (nontemporal) while experts hold at most 48
+// routed tokens on average, i.e. mostly one token tile reads them: E = 128 366 -> 347 us at 400 tokens, 431
+// -> 423 at 1021, 480 -> 470 at 1500, E = 32 138 -> 130 at 256; beyond, the next tiles' reads from L2 win (587 /
+// 651 us at E = 128, 2048 tokens, 188 / 189 at E = 32, 512).
+constexpr uint64_t kGemmStreamPerExpert = 48;
 inline bool use_mx_gemm(const burnext_moe_layer &L, uint64_t n, bool xb) {
   return xb && n >= kMxMinTokens && n * L.K >= kMxMinPerExpert * L.E;
 }
@@ -842,7 +847,7 @@ burnext_status forward_gemm(burnext_moe_layer *L, const void *x, bool xb, uint64
     const uint64_t grid = align_up((uint64_t)g.nrb * max_tiles, 8);
     if (grid > 0x7fffffffull) return fail(BURNEXT_UNSUPPORTED, "expert GEMM grid too large");
     ProfScope ps(L, s, up ? kKGateUp : kKDown);
-    st = check_launch(launch_gemm(g, up != 0, (uint32_t)grid, s), up ? "gate_up GEMM launch" : "down GEMM launch");
+    st = check_launch(launch_gemm(g, up != 0, n * L->K <= kGemmStreamPerExpert * L->E, (uint32_t)grid, s), up ? "gate_up GEMM launch" : "down GEMM launch");
     if (st != BURNEXT_OK) return st;
   }
   return BURNEXT_OK;
@@ -994,13 +999,13 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
   const int nt = xnb ? 1 : 2;
   FusedGeom fg{};
   const bool fused_experts = (flags & BURNEXT_FUSED_EXPERTS) && use_fused(*L, n, nt, pn != nullptr, fg);
-  // a single token that touches few experts runs the expert GEMVs and routes inside the gate_up
-  // launch (route_one_token: no routing launch); other batches run as tiles
-  const bool route1 = n == 1 && !fused_experts && gate_up_split(*L, n);
-  // its down row tiles' K range in fixed parts of whole K-groups (separate work units), as many as
-  // the workspace holds
+  // a single token runs the expert GEMVs and routes inside the gate_up launch (route_one_token: no
+  // routing launch); other batches run as tiles
+  const bool route1 = n == 1 && !fused_experts, up_split = gate_up_split(*L, n);
+  // the down row tiles' K range in fixed parts of whole K-groups (separate work units; few touched
+  // experts: kDownSplitFew parts), as many as the workspace holds
   const uint32_t nkg2 = (L->w2.nb + 3u) / 4u;
-  const uint32_t ksplit = !route1 ? 1u : nkg2 >= kDownSplitFew ? kDownSplitFew : nkg2 >= kDownSplit ? kDownSplit : 1u;
+  const uint32_t ksplit = !route1 ? 1u : up_split && nkg2 >= kDownSplitFew ? kDownSplitFew : nkg2 >= kDownSplit ? kDownSplit : 1u;
   st = pa             ? run_router_front(L, *pa, n, norm, p.rms, p.logits, p.xn, xnb, s)
        : small_router ? run_router_small(L, x, xb, n, norm, p.rms, p.logits, p.xn, xnb && !xb, s)
                       : run_router(L, x, xb, n, norm, p.rms, p.logits, p.xn, s, nullptr, xnb && !xb);
@@ -1017,7 +1022,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
   }
 
   auto gemv = [&](bool gate_up) -> burnext_status {
-    const GemvCfg cf = gemv_cfg(*L, nt, gate_up);
+    const GemvCfg cf = gemv_cfg(*L, nt, gate_up, up_split);
     const TiledMx &t = gate_up ? L->w1 : L->w2;
     GemvArgs g{};
     g.wb = t.blocks;
@@ -1048,7 +1053,7 @@ burnext_status forward_impl(burnext_moe_layer *L, const void *x, burnext_dtype x
       g.ksplit = ksplit;
       g.out_half = n * L->K * L->Dp;
     }
-    if (gate_up) g.ksplit = kGateUpSplit;  // K-parts on the waves of a workgroup, summed there
+    if (gate_up && up_split) g.ksplit = kGateUpSplit;  // K-parts on the waves of a workgroup, summed there
     if (gate_up) {
       g.route1_lg = p.logits;
       g.route1_E = L->E;

@@ -1,6 +1,6 @@
 // tile_gemm.hip -- grouped expert GEMM on bf16 MFMA with MXFP4 weights dequantised in registers: the
-// expert projections of every f32 batch, and of the bf16 batches too small for gemm.hip, but the single
-// tokens that run the expert GEMV (kernels.hip).
+// expert projections of every f32 batch, and of the bf16 batches too small for gemm.hip, but single
+// tokens (the expert GEMV, kernels.hip).
 //
 // replaces w1_swiglu_dense_kernel / w2_scatter_dense_kernel (src/quant/gpu.rs:89-192) for those
 // batches (the reference runs them per 256-token tile and per used expert, src/moe/mod.rs:262-404).

@@ -23,6 +23,12 @@ TOL = {"f32": 1e-4, "bf16": 2e-2}
     (50, 31, 6, 2, 60, "bf16", "halves", 0),           # odd F: the last value of a row segment alone
     (2880, 2880, 128, 4, 63, "bf16", "interleaved", 3),
     (2880, 2880, 32, 4, 17, "bf16", "interleaved", 3),
+    # the grouped GEMM at both sides of its first sizes and of its tiles of 2, 3 and 4 token columns
+    (256, 256, 1, 1, 79, "bf16", "interleaved", 3),
+    (256, 256, 1, 1, 96, "bf16", "interleaved", 3),
+    (256, 256, 1, 1, 112, "bf16", "interleaved", 3),
+    (640, 1152, 3, 1, 97, "bf16", "interleaved", 3),
+    (2200, 520, 2, 2, 97, "bf16", "halves", 3),
     # decode sizes: one tile of up to 16 tokens per active expert
     (256, 256, 2, 2, 16, "f32", "interleaved", 3),     # full tiles
     (200, 100, 3, 3, 2, "bf16", "halves", 3),          # partial K-groups
