@@ -846,43 +846,95 @@ struct LogitsArgs {
   int32_t *bidx;  // [B][nblk]
 };
 
-__device__ __forceinline__ void block_best(float &bv, int32_t &bi, float *rv, int32_t *ri) {
-  const uint32_t t = threadIdx.x;
-  rv[t] = bv;
-  ri[t] = bi;
-  __syncthreads();
-  for (uint32_t st = 128; st >= 1; st >>= 1) {
-    if (t < st && ri[t + st] != kNoIndex && (ri[t] == kNoIndex || beats(rv[t + st], ri[t + st], rv[t], ri[t]))) {
-      rv[t] = rv[t + st];
-      ri[t] = ri[t + st];
-    }
-    __syncthreads();
+// (bv, bi) <- the better of it and lane (lane ^ m)'s (`beats`; kNoIndex for none)
+__device__ __forceinline__ void best_xor(float &bv, int32_t &bi, int m) {
+  const float ov = __shfl_xor(bv, m, 64);
+  const int32_t oi = __shfl_xor(bi, m, 64);
+  if (oi != kNoIndex && (bi == kNoIndex || beats(ov, oi, bv, bi))) {
+    bv = ov;
+    bi = oi;
   }
-  bv = rv[0];
-  bi = ri[0];
 }
 
+// The best entry of the 4 waves of a workgroup, in thread 0.
+__device__ __forceinline__ void block_best(float &bv, int32_t &bi) {
+  __shared__ float wbv[4];
+  __shared__ int32_t wbi[4];
+  const uint32_t t = threadIdx.x;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) best_xor(bv, bi, m);
+  if ((t & 63u) == 0u) {
+    wbv[t >> 6] = bv;
+    wbi[t >> 6] = bi;
+  }
+  __syncthreads();
+  if (t == 0u)
+#pragma unroll
+    for (uint32_t w = 1; w < 4u; ++w)
+      if (wbi[w] != kNoIndex && (bi == kNoIndex || beats(wbv[w], wbi[w], bv, bi))) {
+        bv = wbv[w];
+        bi = wbi[w];
+      }
+}
+
+// P > 0: exactly P parts, all of a thread's P values of 4 rows requested before the first sum (a
+// loop over a run-time part count waits for part after part, row after row: 9.8 -> 4.9 us at 16 x 16384
+// logits of 6 parts); P = 0: a.parts parts in a loop.
+template <uint32_t P>
 __global__ __launch_bounds__(256) void logits_kernel(LogitsArgs a) {
-  __shared__ float rv[256];
-  __shared__ int32_t ri[256];
-  const uint32_t b = blockIdx.y, t = threadIdx.x;
+  constexpr uint32_t U = kLogitsPerBlock / 256u;
+  const uint32_t b = blockIdx.y, t = threadIdx.x, v0 = blockIdx.x * kLogitsPerBlock + t;
+  const float *pb = a.part + (size_t)b * a.V;
+  float s[U];
+  if constexpr (P > 0) {
+    float pv[U][P];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+#pragma unroll
+      for (uint32_t h = 0; h < P; ++h) pv[u][h] = pb[(size_t)h * a.part_stride + min(v0 + u * 256u, a.V - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      s[u] = 0.0f;
+#pragma unroll
+      for (uint32_t h = 0; h < P; ++h) s[u] = s[u] + pv[u][h];
+    }
+  } else {
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) s[u] = 0.0f;
+    for (uint32_t h = 0; h < a.parts; ++h)
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) s[u] = s[u] + pb[(size_t)h * a.part_stride + min(v0 + u * 256u, a.V - 1u)];
+  }
   float bv = -INFINITY;
   int32_t bi = kNoIndex;
-  for (uint32_t u = 0; u < kLogitsPerBlock / 256u; ++u) {
-    const uint32_t v = blockIdx.x * kLogitsPerBlock + u * 256u + t;
-    if (v >= a.V) break;
-    float s = 0.0f;
-    for (uint32_t h = 0; h < a.parts; ++h) s = s + a.part[(size_t)h * a.part_stride + (size_t)b * a.V + v];
-    if (a.logits) a.logits[(size_t)b * a.V + v] = s;
-    if (bi == kNoIndex || beats(s, (int32_t)v, bv, bi)) {
-      bv = s;
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) {
+    const uint32_t v = v0 + u * 256u;
+    if (v >= a.V) continue;
+    if (a.logits) a.logits[(size_t)b * a.V + v] = s[u];
+    if (bi == kNoIndex || beats(s[u], (int32_t)v, bv, bi)) {
+      bv = s[u];
       bi = (int32_t)v;
     }
   }
-  block_best(bv, bi, rv, ri);
+  block_best(bv, bi);
   if (t == 0) {
     a.bval[(size_t)b * a.nblk + blockIdx.x] = bv;
     a.bidx[(size_t)b * a.nblk + blockIdx.x] = bi;
+  }
+}
+
+hipError_t launch_logits(const LogitsArgs &a, dim3 grid, hipStream_t s) {
+  switch (a.parts) {  // the part counts dense_plan gives at d_model <= 4096
+    case 1: return launch_kernel(logits_kernel<1>, grid, dim3(256), 0, s, a);
+    case 2: return launch_kernel(logits_kernel<2>, grid, dim3(256), 0, s, a);
+    case 3: return launch_kernel(logits_kernel<3>, grid, dim3(256), 0, s, a);
+    case 4: return launch_kernel(logits_kernel<4>, grid, dim3(256), 0, s, a);
+    case 5: return launch_kernel(logits_kernel<5>, grid, dim3(256), 0, s, a);
+    case 6: return launch_kernel(logits_kernel<6>, grid, dim3(256), 0, s, a);
+    case 7: return launch_kernel(logits_kernel<7>, grid, dim3(256), 0, s, a);
+    case 8: return launch_kernel(logits_kernel<8>, grid, dim3(256), 0, s, a);
+    default: return launch_kernel(logits_kernel<0>, grid, dim3(256), 0, s, a);
   }
 }
 
@@ -893,8 +945,6 @@ struct ArgmaxArgs {
   int32_t *next;
 };
 __global__ __launch_bounds__(256) void argmax_kernel(ArgmaxArgs a) {
-  __shared__ float rv[256];
-  __shared__ int32_t ri[256];
   const uint32_t b = blockIdx.x, t = threadIdx.x;
   float bv = -INFINITY;
   int32_t bi = kNoIndex;
@@ -906,7 +956,7 @@ __global__ __launch_bounds__(256) void argmax_kernel(ArgmaxArgs a) {
       bi = ix;
     }
   }
-  block_best(bv, bi, rv, ri);
+  block_best(bv, bi);
   if (t == 0) a.next[b] = bi;
 }
 
@@ -943,16 +993,6 @@ struct LmArgs {
   uint32_t iq, ir;   // iters = iq W + ir
   uint32_t V, K, nkg, B, W, nblk, nblk_s;
 };
-
-// (bv, bi) <- the better of it and lane (lane ^ m)'s (`beats`; kNoIndex for none)
-__device__ __forceinline__ void best_xor(float &bv, int32_t &bi, int m) {
-  const float ov = __shfl_xor(bv, m, 64);
-  const int32_t oi = __shfl_xor(bi, m, 64);
-  if (oi != kNoIndex && (bi == kNoIndex || beats(ov, oi, bv, bi))) {
-    bv = ov;
-    bi = oi;
-  }
-}
 
 __global__ __launch_bounds__(kLmWaves * 64) void lm_stream_kernel(LmArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1267,14 +1307,15 @@ struct GWs {
 
 // The streaming LM head (lm_stream_kernel) serves batches of at most kLmMaxB rows whose d_model
 // fits its LDS staging (K <= kLmMaxK, K % 8 == 0, a batch of at least 1 KiB for the dummy refills)
-// and vocabularies that give at least half the CUs a workgroup (a wave takes at least one row tile:
-// 16 384 rows are 64 workgroups), with fewer than 2^32 K-groups (lm_fix_kernel's 32-bit cuts).
-// Decode steps with it against the K-split GEMV, d_model 2880, 1 / 8 rows: 96 / 108 against 85 / 95 us at
-// 16 384, 102 / 112 and 99 / 112 at 32 768, 112 / 125 and 114 / 134 at 50 001, 157 / 173 and 158 / 186 at 100 000.
+// and vocabularies that give at least three quarters of the CUs a workgroup (a wave takes at least
+// one row tile: 16 384 rows are 64 workgroups), with fewer than 2^32 K-groups (lm_fix_kernel's 32-bit
+// cuts).  Decode steps with it against the K-split GEMV, d_model 2880, 1 / 8 rows: 96 / 107 against 78 / 90 us
+// at 16 384, 101 / 112 and 92 / 107 at 32 768, 112 / 125 and 108 / 128 at 50 001, 155 / 173 and 151 / 183 at
+// 100 000.
 bool lm_stream_ok(const burnext_gptoss &M, uint32_t B) {
   const uint32_t K = M.lm.K;
   return B >= 1u && B <= kLmMaxB && K <= kLmMaxK && K % 8u == 0u && (uint64_t)B * K * 4u >= 1024u &&
-         2ull * M.lm.ntiles >= (uint64_t)kLmWaves * (uint32_t)M.num_cus && (uint64_t)M.lm.ntiles * M.lm.nkg < (1ull << 32);
+         4ull * M.lm.ntiles >= 3ull * kLmWaves * (uint32_t)M.num_cus && (uint64_t)M.lm.ntiles * M.lm.nkg < (1ull << 32);
 }
 // Its waves: one workgroup per CU, at most one wave per row tile (so every run spans at least nkg
 // K-groups and a tile is cut at most once).
@@ -1854,7 +1895,7 @@ burnext_status burnext_gptoss_decode(burnext_gptoss_t M, const int32_t *tokens, 
     st = dense_gemv(M->lm, xn, B, part, s);
     if (st != BURNEXT_OK) return st;
     LogitsArgs la{part, (uint64_t)B * c.vocab_size, M->lm.parts, c.vocab_size, w.nblk, logits, bval, bidx};
-    st = hip_check(launch_kernel(logits_kernel, dim3(w.nblk, B), dim3(256), 0, s, la), "logits launch");
+    st = hip_check(launch_logits(la, dim3(w.nblk, B), s), "logits launch");
     if (st != BURNEXT_OK) return st;
   }
   ArgmaxArgs ga{bval, bidx, w.nblk, next_tokens};
