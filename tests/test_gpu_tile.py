@@ -1,5 +1,5 @@
-"""GPU: the expert projections as tiles on bf16 MFMA (all batches but single tokens on few experts and
-those of the grouped GEMM) against the oracle on every row: token tiles of 1..64 rows, row blocks and K-groups with
+"""GPU: the expert projections as tiles on bf16 MFMA (all batches but single tokens and those of the
+grouped GEMM) against the oracle on every row: token tiles of 1..64 rows, row blocks and K-groups with
 remainders, one and several tiles per expert.  Bars as the other forwards': f32 rows 1e-4 (two bf16
 terms, 2^-17 per value), bf16 rows 2e-2."""
 import numpy as np
@@ -36,7 +36,7 @@ TOL = {"f32": 1e-4, "bf16": 2e-2}
     (640, 1152, 256, 8, 7, "bf16", "interleaved", 1),  # the most experts
     (50, 31, 6, 2, 11, "f32", "interleaved", 0),
     (2880, 2880, 32, 4, 2, "f32", "interleaved", 3),
-    (1024, 2048, 64, 16, 1, "bf16", "interleaved", 3), # one token on too many experts for the GEMVs
+    (1024, 2048, 64, 16, 1, "bf16", "interleaved", 3), # one token: the GEMVs, without K-parts in gate_up
 ])
 def test_forward_tiles_all_rows(oracle, D, F, E, K, n, dtype, layout, flags):
     from burnext_amd import moe, synth
