@@ -2074,31 +2074,41 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(CombineArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Dequant hook.  Bound by its output stores, so the work is split by output: a thread makes the
-// 16 bytes of one store (8 bf16 or 4 f32 consecutive values of the flat [rows * cols] output),
-// kDequantUnroll stores per thread, consecutive lanes on consecutive 16 bytes, all source loads of
-// a thread requested before its first convert.  One thread per packed byte (two 2- or 4-byte stores
+// Dequant hook.  Bound by its output stores, so the work is split by output: a thread makes 16-byte
+// stores of consecutive values of the flat [rows * cols] output (8 bf16, 4 f32; MODE 2: 8 f32 in two),
+// 4 of them, consecutive lanes on consecutive pieces, all source loads of a thread
+// requested before its first convert.  One thread per packed byte (two 2- or 4-byte stores
 // and a 64-bit division each) took 175 us for 8 x 5760 x 2880 to bf16 (336 MB), this 64 us.
 // f32 output uses the bit-built LUT value times the bit-built 2^(s-127); bf16 output uses the same
 // v_cvt_scalef32_pk_bf16_fp4 conversion as the expert projections, so the exhaustive test of this
 // hook covers their dequantisation.
 // MODE 0: cols a multiple of 8 (a thread's values lie in one 32-value block); 1: cols even (the
-// packed rows are one contiguous nibble stream, pairs never cross a row or a block); 2: any cols
-// and any alignment (value by value).  0 and 1 need blocks 4-byte and out 16-byte aligned.  Each mode
-// only where the one before cannot go (8 x 5760 rows, bf16 / f32): 2880 columns 67 / 125 us in mode 0
-// and 152 / 200 in mode 2; 2818 columns 71 / 130 us in mode 1 and 146 / 195 in mode 2.
+// packed rows are one contiguous nibble stream, pairs never cross a row or a block); both need blocks
+// 4-byte and out 16-byte aligned.  2: any cols from 8 on and any alignment: 8 values touch at most two rows
+// and three blocks, so an (unaligned) 8-byte load at the first value, one at the next row's start and
+// three scale bytes serve them.  3: rows of fewer than 8 values, value by value.
+// MODE 2 at 40000 x 2879, bf16 / f32: 84 / 146 us, value by value 122 / 172, one thread per byte 161 / 226;
+// at 9600 x 2879 22 / 26, value by value 32 / 37, one thread per byte 28 / 33.
+// Each mode only where the one before cannot go (40000 x 2880 in mode 0 55 / 109 us).
 // ---------------------------------------------------------------------------------------------
-constexpr uint32_t kDequantUnroll = 4;
+// values per store step of a thread, and steps
+constexpr uint32_t dequant_vals(bool bf16, int mode) { return bf16 || mode == 2 ? 8u : 4u; }
+constexpr uint32_t dequant_unroll(int mode) { return mode == 2 ? 2u : 4u; }
 
 template <bool BF16, int MODE>
 __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
-  constexpr uint32_t V = BF16 ? 8u : 4u, U = kDequantUnroll, kSpan = 256u * V * U;
-  constexpr uint32_t NS = MODE == 0 ? 1u : MODE == 1 ? V / 2u : V;  // scales (and, MODE 2, bytes) per store
+  constexpr uint32_t V = dequant_vals(BF16, MODE), U = dequant_unroll(MODE), kSpan = 256u * V * U;
+  constexpr uint32_t W = BF16 ? V / 2u : V;  // output dwords per step
+  constexpr uint32_t NS = MODE == 0 ? 1u : MODE == 1 ? V / 2u : MODE == 2 ? 3u : V;  // scales (and, MODE 3, bytes) per store
+  typedef uint64_t u64_any __attribute__((aligned(1)));
+  const uint64_t nbytes = a.rows * a.bpr;
   const uint64_t total = a.rows * a.cols;
   const bool wide = a.cols > 0x7fffffffull;  // then a span crosses at most one row end
   for (uint64_t base = (uint64_t)blockIdx.x * kSpan; base < total; base += (uint64_t)gridDim.x * kSpan) {
     const uint64_t r0 = base / a.cols, c0 = base - r0 * a.cols;
     uint32_t w[U], by[U][NS], sb[U][NS];
+    uint64_t lo[U], hi[U];      // MODE 2: the 8 bytes at the store's first value and at its next row's start
+    uint32_t n1[U], sh[U], sq[U], c5[U];  // values on the first row, bit offsets in lo and hi, column mod 32
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) {
       // the store's first value (clamped into the output: the last span's surplus lanes reload it)
@@ -2107,7 +2117,23 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
       const uint64_t dr = wide ? (uint64_t)(o >= a.cols) : (uint64_t)((uint32_t)o / (uint32_t)a.cols);
       uint64_t r = r0 + dr, c = o - dr * a.cols;
       w[u] = 0u;
-      if constexpr (MODE != 2) {
+      if constexpr (MODE == 2) {
+        // loads end at the packed matrix's last byte at the latest: shifted instead
+        n1[u] = (uint32_t)min((uint64_t)V, a.cols - c);
+        const uint64_t rn = n1[u] < V && r + 1u < a.rows ? r + 1u : r;
+        const uint64_t pb = r * a.bpr + (c >> 1), qb = rn > r ? rn * a.bpr : pb;
+        const uint64_t pa = min(pb, nbytes - 8u), qa = min(qb, nbytes - 8u);
+        lo[u] = *(const u64_any *)(a.blocks + pa);
+        hi[u] = *(const u64_any *)(a.blocks + qa);
+        sh[u] = 8u * (uint32_t)(pb - pa) + 4u * (uint32_t)(c & 1u);
+        sq[u] = 8u * (uint32_t)(qb - qa);
+        c5[u] = (uint32_t)c & 31u;
+        sb[u][0] = a.scales[r * a.gpr + (c >> 5)];
+        sb[u][1] = a.scales[r * a.gpr + ((c + n1[u] - 1u) >> 5)];
+        sb[u][2] = a.scales[rn * a.gpr + (rn > r ? 0u : c >> 5)];
+        continue;
+      }
+      if constexpr (MODE < 2) {
         if (f + V <= total) {
           w[u] = BF16 ? *(const uint32_t *)(a.blocks + f / 2u) : (uint32_t)*(const uint16_t *)(a.blocks + f / 2u);
         } else {
@@ -2119,7 +2145,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
 #pragma unroll
       for (uint32_t e = 0; e < NS; ++e) {
         sb[u][e] = a.scales[r * a.gpr + (c >> 5)];
-        if constexpr (MODE == 2) by[u][e] = (uint32_t)a.blocks[r * a.bpr + (c >> 1)] >> (4u * (uint32_t)(c & 1u));
+        if constexpr (MODE == 3) by[u][e] = (uint32_t)a.blocks[r * a.bpr + (c >> 1)] >> (4u * (uint32_t)(c & 1u));
         c += MODE == 1 ? 2u : 1u;
         if (c >= a.cols) {  // next row (the last value's successor stays on it)
           if (r + 1u < a.rows) {
@@ -2135,17 +2161,26 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
     for (uint32_t u = 0; u < U; ++u) {
       const uint64_t f = base + (u * 256u + threadIdx.x) * V;
       if (f >= total) continue;
-      uint32_t out[4];
+      uint32_t out[W];
       auto scale = [&](uint32_t e) {  // of value e of the store
-        const uint32_t s = sb[u][MODE == 0 ? 0u : MODE == 1 ? e / 2u : e];
+        uint32_t s;
+        if constexpr (MODE == 2)
+          s = e >= n1[u] ? sb[u][2] : c5[u] + e < 32u ? sb[u][0] : sb[u][1];
+        else
+          s = sb[u][MODE == 0 ? 0u : MODE == 1 ? e / 2u : e];
         return e8m0_to_f32((s - (uint32_t)a.ue8_offset) & 255u);
       };
+      if constexpr (MODE == 2)
+        w[u] = (uint32_t)(((lo[u] >> sh[u]) & ((1ull << (4u * n1[u])) - 1ull)) | ((hi[u] >> sq[u]) << (4u * n1[u])));
       if constexpr (BF16) {
-        if constexpr (MODE == 2) {
+        if constexpr (MODE >= 2) {
+          uint32_t nib[V];
+#pragma unroll
+          for (uint32_t e = 0; e < V; ++e) nib[e] = MODE == 3 ? by[u][e % NS] : w[u] >> (4u * e);
 #pragma unroll
           for (uint32_t j = 0; j < 4u; ++j)
-            out[j] = (fp4x2_to_bf16x2_bits<0>(by[u][2u * j] & 15u, scale(2u * j)) & 0xFFFFu) |
-                     (fp4x2_to_bf16x2_bits<0>(by[u][2u * j + 1u] & 15u, scale(2u * j + 1u)) << 16);
+            out[j] = (fp4x2_to_bf16x2_bits<0>(nib[2u * j] & 15u, scale(2u * j)) & 0xFFFFu) |
+                     (fp4x2_to_bf16x2_bits<0>(nib[2u * j + 1u] & 15u, scale(2u * j + 1u)) << 16);
         } else {
           out[0] = fp4x2_to_bf16x2_bits<0>(w[u], scale(0));
           out[1] = fp4x2_to_bf16x2_bits<1>(w[u], scale(2));
@@ -2154,11 +2189,13 @@ __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
         }
       } else {
 #pragma unroll
-        for (uint32_t j = 0; j < 4u; ++j)
-          out[j] = __float_as_uint(fp4_to_f32((MODE == 2 ? by[u][j] : w[u] >> (4u * j)) & 15u) * scale(j));
+        for (uint32_t j = 0; j < V; ++j)
+          out[j] = __float_as_uint(fp4_to_f32((MODE == 3 ? by[u][j % NS] : w[u] >> (4u * j)) & 15u) * scale(j));
       }
-      if (f + V <= total && (MODE != 2 || a.vec)) {
-        *(uint4 *)((uint8_t *)a.out + f * (16u / V)) = make_uint4(out[0], out[1], out[2], out[3]);
+      if (f + V <= total && (MODE < 2 || a.vec)) {
+#pragma unroll
+        for (uint32_t j = 0; j < W; j += 4u)
+          *(uint4 *)((uint8_t *)a.out + f * (BF16 ? 2u : 4u) + 4u * j) = make_uint4(out[j], out[j + 1u], out[j + 2u], out[j + 3u]);
       } else {
 #pragma unroll
         for (uint32_t e = 0; e < V; ++e) {
@@ -2438,17 +2475,20 @@ hipError_t launch_dequant(const DequantArgs &args, hipStream_t s) {
   DequantArgs a = args;
   if (a.rows * a.cols == 0) return hipSuccess;
   a.vec = ((uintptr_t)a.out & 15u) == 0;
-  const int mode = !a.vec || ((uintptr_t)a.blocks & 3u) != 0 || a.cols % 2u != 0 ? 2 : a.cols % 8u != 0 ? 1 : 0;
-  const uint64_t span = 256u * (a.out_bf16 ? 8u : 4u) * kDequantUnroll;
+  const int mode = !a.vec || ((uintptr_t)a.blocks & 3u) != 0 || a.cols % 2u != 0 ? (a.cols >= 8u && a.rows * a.bpr >= 8u ? 2 : 3)
+                   : a.cols % 8u != 0 ? 1 : 0;
+  const uint64_t span = 256u * dequant_vals(a.out_bf16 != 0, mode) * dequant_unroll(mode);
   const dim3 grid((uint32_t)std::min<uint64_t>((a.rows * a.cols + span - 1u) / span, 1u << 20)), block(256);
   if (a.out_bf16)
     (void)(mode == 0   ? launch_kernel(dequant_kernel<true, 0>, grid, block, 0, s, a)
            : mode == 1 ? launch_kernel(dequant_kernel<true, 1>, grid, block, 0, s, a)
-                       : launch_kernel(dequant_kernel<true, 2>, grid, block, 0, s, a));
+           : mode == 2 ? launch_kernel(dequant_kernel<true, 2>, grid, block, 0, s, a)
+                       : launch_kernel(dequant_kernel<true, 3>, grid, block, 0, s, a));
   else
     (void)(mode == 0   ? launch_kernel(dequant_kernel<false, 0>, grid, block, 0, s, a)
            : mode == 1 ? launch_kernel(dequant_kernel<false, 1>, grid, block, 0, s, a)
-                       : launch_kernel(dequant_kernel<false, 2>, grid, block, 0, s, a));
+           : mode == 2 ? launch_kernel(dequant_kernel<false, 2>, grid, block, 0, s, a)
+                       : launch_kernel(dequant_kernel<false, 3>, grid, block, 0, s, a));
   return hipGetLastError();
 }
 

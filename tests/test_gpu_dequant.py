@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(1, 1), (1, 7), (3, 8), (5, 2), (37, 30), (33, 31), (9, 32), (65, 33), (70, 1000),
-                                       (11, 2818), (7, 2817), (13, 4104)])
+                                       (1, 8), (1, 9), (2, 11), (5, 15), (301, 129), (11, 2818), (7, 2817), (13, 4104)])
 def test_dequant_shapes(oracle, rows, cols, out_dtype):
     from burnext_amd import _native as N
     from burnext_amd import moe
