@@ -20,7 +20,8 @@
 // in the 32-token shape only (gate_up 58 -> 50 us at 45 tokens: the router rows and token rows stay in
 // the caches); the 64-token shape re-reads them from L2 for the next tiles.  At decode sizes the
 // short items refill the CUs as they end, where the GEMV's fixed shares waited for the slowest: 8 tokens
-// 38 + 22 -> 35 + 19 us, 16 tokens in f32 64 + 33 -> 52 + 27 us, D = F = 256 with 16 tokens 14 + 13 -> 7 + 7 us
+// 38 + 22 -> 35 + 19 us with one layer's weights (over four layers in turn, which no cache holds, the step
+// 75.5 -> 73.9 us), 16 tokens in f32 64 + 33 -> 52 + 27 us, D = F = 256 with 16 tokens 14 + 13 -> 7 + 7 us
 // (every prefix and segment entry an item needs comes in one round trip, and waves whose token
 // columns are all empty skip the split).
 #include <type_traits>
