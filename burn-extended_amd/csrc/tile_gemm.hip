@@ -17,7 +17,7 @@
 // weight stream: 17 tokens gate_up 54 -> 47 us (283 MB, 6.0 TB/s), down 30 -> 26 us.  Large f32 batches are
 // bound by the matrix cores: 523 tokens 793 + 423 -> 182 + 117 us, 4096 tokens 918 + 483 us (1.16
 // PFLOP/s of the two terms' products; plain bf16 MFMAs reach 1.8).  Weights are read nontemporally
-// in the 32-token shape only (gate_up 58 -> 50 us at 45 tokens: the router rows and token rows stay in
+// in the 16- and 32-token shapes only (gate_up 58 -> 50 us at 45 tokens: the router rows and token rows stay in
 // the caches); the 64-token shape re-reads them from L2 for the next tiles.  At decode sizes the
 // short items refill the CUs as they end, where the GEMV's fixed shares waited for the slowest: 8 tokens
 // 38 + 22 -> 35 + 19 us with one layer's weights (over four layers in turn, which no cache holds, the step
